@@ -350,6 +350,18 @@ int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv
                       int partition_tiles, int32_t* items, int64_t items_capacity,
                       int32_t* merges, int64_t merges_capacity, int64_t* counts);
 
+/* mf_attention_plan for a device of `num_cus` compute units
+ * (hipDeviceProp_t::multiProcessorCount), with the partitions chosen by the
+ * planner: the same records, run by the same entry points, with the same
+ * results up to fp32 summation order. Wide workgroups (16-bit types, head_dim
+ * a kernel size) are cut by column quads, for about two or four workgroups per
+ * compute unit, with ranges of any length. No counterpart
+ * in the reference: it serves the launch, not the data path. */
+int mf_attention_plan_device(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
+                             int num_q_heads, int num_kv_heads, int head_dim, int dtype, int num_cus,
+                             int32_t* items, int64_t items_capacity, int32_t* merges,
+                             int64_t merges_capacity, int64_t* counts);
+
 /* ------------------------------------------------- decode slice plans
  * A second plan form for large decode launches, with the same results as
  * mf_attention_plan + mf_paged_attention (up to fp32 summation order).

@@ -75,6 +75,8 @@ _SIGNATURES = {
         _c_int, _c_f32, _vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _vp]),
     "mf_attention_plan": (_c_int, [_c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int,
                                    _vp, _c_i64, _vp, _c_i64, _vp]),
+    "mf_attention_plan_device": (_c_int, [_c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                          _vp, _c_i64, _vp, _c_i64, _vp]),
     "mf_attention_plan_slices": (_c_int, [_c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int,
                                           _c_int, _vp, _c_i64, _vp, _c_i64, _vp]),
     "mf_paged_attention_slices": (_c_int, [
@@ -404,9 +406,11 @@ class AttentionPlan:
 
 def plan_attention_host(cu_seqlens: Sequence[int], kv_lens: Sequence[int], num_q_heads: int,
                         num_kv_heads: int, head_dim: int, dtype: torch.dtype,
-                        partition_tiles: int = 0) -> Tuple[np.ndarray, np.ndarray, np.ndarray]:
+                        partition_tiles: int = 0, num_cus: int = 0) -> Tuple[np.ndarray, np.ndarray, np.ndarray]:
     """mf_attention_plan on host arrays: (items [n, PLAN_ITEM_INTS], merges
-    [m, PLAN_MERGE_INTS], counts [n_narrow, n_wide, n_merges, partials_floats])."""
+    [m, PLAN_MERGE_INTS], counts [n_narrow, n_wide, n_merges, partials_floats]).
+    With ``num_cus`` and no ``partition_tiles``, mf_attention_plan_device: the
+    ranges cut for a GPU of that many compute units."""
     cu = np.ascontiguousarray(np.asarray(cu_seqlens, dtype=np.int32))
     kv = np.ascontiguousarray(np.asarray(kv_lens, dtype=np.int32))
     B = kv.shape[0]
@@ -414,24 +418,24 @@ def plan_attention_host(cu_seqlens: Sequence[int], kv_lens: Sequence[int], num_q
         raise ValueError("cu_seqlens must have one more entry than kv_lens")
     counts = np.zeros(4, dtype=np.int64)
     L = lib()
-    args = (B, cu.ctypes.data, kv.ctypes.data, num_q_heads, num_kv_heads, head_dim,
-            dtype_code(dtype), partition_tiles)
+    args = [B, cu.ctypes.data, kv.ctypes.data, num_q_heads, num_kv_heads, head_dim, dtype_code(dtype)]
+    device = num_cus > 0 and partition_tiles <= 0
+    plan = L.mf_attention_plan_device if device else L.mf_attention_plan
+    args.append(num_cus if device else partition_tiles)
     # One planner call when the plan fits the largest one seen so far (the
     # planner fills every row it reports); otherwise it reports the sizes and
     # a second call fills arrays of exactly that size.
     cap_items, cap_merges = _PLAN_CAPACITY
     items = np.empty((cap_items, PLAN_ITEM_INTS), dtype=np.int32)
     merges = np.empty((cap_merges, PLAN_MERGE_INTS), dtype=np.int32)
-    st = L.mf_attention_plan(*args, items.ctypes.data, cap_items, merges.ctypes.data, cap_merges,
-                             counts.ctypes.data)
+    st = plan(*args, items.ctypes.data, cap_items, merges.ctypes.data, cap_merges, counts.ctypes.data)
     if st == -3:  # MF_ERR_WORKSPACE: counts holds the sizes
         n_items, n_merges = int(counts[0] + counts[1]), int(counts[2])
         _PLAN_CAPACITY[0] = max(cap_items, min(n_items, 1 << 16))
         _PLAN_CAPACITY[1] = max(cap_merges, min(n_merges, 1 << 14))
         items = np.empty((max(n_items, 1), PLAN_ITEM_INTS), dtype=np.int32)
         merges = np.empty((max(n_merges, 1), PLAN_MERGE_INTS), dtype=np.int32)
-        st = L.mf_attention_plan(*args, items.ctypes.data, n_items, merges.ctypes.data, n_merges,
-                                 counts.ctypes.data)
+        st = plan(*args, items.ctypes.data, n_items, merges.ctypes.data, n_merges, counts.ctypes.data)
     _check(st, "mf_attention_plan")
     n_items = int(counts[0] + counts[1])
     n_merges = int(counts[2])
@@ -515,10 +519,11 @@ def plan_host(cu_seqlens: Sequence[int], kv_lens: Sequence[int], num_q_heads: in
     blocks, no row map and no in-flight keys) a decode step large enough to
     fill the GPU on ``device`` more than once gets a slice plan; every other
     call, and an explicit ``partition_tiles``, the per-range plan."""
-    slices = decode_slices and partition_tiles <= 0 and device is not None and torch.device(device).type == "cuda"
-    cus = device_cus(device) if slices else 0
+    on_gpu = partition_tiles <= 0 and device is not None and torch.device(device).type == "cuda"
+    slices = decode_slices and on_gpu
+    cus = device_cus(device) if on_gpu else 0
     key = (tuple(int(x) for x in cu_seqlens), tuple(int(x) for x in kv_lens), num_q_heads, num_kv_heads,
-           head_dim, dtype, partition_tiles, cus)
+           head_dim, dtype, partition_tiles, cus, slices)
     hit = _PLAN_CACHE.get(key)
     if hit is not None:
         _PLAN_CACHE.move_to_end(key)
@@ -528,7 +533,7 @@ def plan_host(cu_seqlens: Sequence[int], kv_lens: Sequence[int], num_q_heads: in
         out = (*made, True)
     else:
         out = (*plan_attention_host(cu_seqlens, kv_lens, num_q_heads, num_kv_heads, head_dim, dtype,
-                                    partition_tiles), False)
+                                    partition_tiles, cus), False)
     for a in out[:3]:
         a.flags.writeable = False
     _PLAN_CACHE[key] = out

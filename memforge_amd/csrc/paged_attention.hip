@@ -15,7 +15,8 @@
 // O^T = V^T P^T with a second MFMA whose B operand is the exponentiated S^T
 // tile exactly as the first MFMA left it in registers. V arrives with
 // fully coalesced 16-token x 16-byte row loads and is transposed into the MFMA
-// A layout with byte permutes; no LDS is used at all.
+// A layout with byte permutes. 16-bit prefill runs in workgroups that share
+// each K/V row through LDS instead (attn_wide_body).
 //
 // Long contexts are split into key partitions (the plan decides); partial
 // (max, sum, unnormalised output) triples go to fp32 scratch and a merge
@@ -49,11 +50,6 @@ constexpr int kWaves = 4;  // waves per workgroup; each wave runs its own item
 constexpr int kMaxItemTiles = MF_MAX_ITEM_TILES;  // key tiles per work item (two block-table entries per lane)
 #ifndef MF_NARROW_ITEMS
 #define MF_NARROW_ITEMS 4096  // planner: target item count that sets the narrow key partition
-#endif
-// Stages of the workgroup-shared prefill loop move global -> LDS directly
-// (1) or through registers (0).
-#ifndef MF_WIDE_DIRECT_LDS
-#define MF_WIDE_DIRECT_LDS 1
 #endif
 // Wave priority (s_setprio) of the workgroup-shared wide loop. In a mixed
 // launch a CU holds single-tile (decode) waves beside the wide (prefill) ones;
@@ -95,11 +91,10 @@ constexpr float kLazyLog2 = 8.f;  // running-max slack of the online softmax (lo
 constexpr float kMinM = -1e30f;
 
 // 16-column tiles one wave carries for multi-tile (prefill / wide verify)
-// items: as many as fit in registers without spilling.
+// items.
 __host__ __device__ constexpr int wide_tiles(int dt, int dp) {
-    // measured on MI355X: 2 tiles beat 4 for 16-bit head_dim 64 (more waves
-    // per SIMD outweigh the K/V reuse across columns)
-    return dt == MF_F32 ? (dp >= 128 ? 2 : 4) : (dp >= 256 ? 1 : (dp == 64 ? 2 : 4));
+    // 16-bit: the 32 columns of one MFMA block (attn_wide_body)
+    return dt == MF_F32 ? (dp >= 128 ? 2 : 4) : (dp >= 256 ? 1 : 2);
 }
 
 struct AttnArgs {
@@ -413,13 +408,37 @@ __device__ __forceinline__ void merge_tile(const AttnArgs& a, const int32_t* mg,
     store_out_chunk<DT, VCH>(a.out + ((int64_t)prow * a.o_sr + (int64_t)qhead * a.o_sh + dbase) * ES, o);
 }
 
+// Fused split-K merge: the last partition of a group to arrive merges the
+// group. Release the partials (agent-scope fence: the L2s of the XCDs are not
+// coherent with each other), count the arrival, and on the last arrival
+// acquire everyone else's partials and reset the counter for the next call.
+// Every wave runs to the end; nothing waits on another wave.
+template <int DT, int DP>
+__device__ __forceinline__ void arrive_and_merge(const AttnArgs& a, int m0, int nct, int lane) {
+    if (a.counters == nullptr) return;
+    __threadfence();
+    int prev = 0;
+    if (lane == 0) prev = atomicAdd(a.counters + m0, 1);
+    prev = __shfl(prev, 0, 64);
+    const int32_t* mg0 = a.merges + (int64_t)m0 * MF_PLAN_MERGE_INTS;
+    if (prev == mg0[3] - 1) {
+        __threadfence();
+        if (lane == 0) a.counters[m0] = 0;
+        for (int o = 0; o < nct; ++o) merge_tile<DT, DP>(a, mg0 + o * MF_PLAN_MERGE_INTS, lane >> 4, lane & 15);
+    }
+}
+
 // -------------------------------------------------------------- main kernel
 // Waves per SIMD the register allocator must leave room for: two where the
 // kernel fits in 256 registers without spilling (key rows up to 128 bytes,
 // or up to 256 bytes for single-tile items), else one.
+#ifndef MF_WIDE_WAVES
+#define MF_WIDE_WAVES(dp) ((dp) == 128 ? 3 : 4)
+#endif
 template <int DT, int DP, int NT>
 constexpr int attn_waves_per_eu() {
     constexpr int row_bytes = DP * (DT == MF_F32 ? 4 : 2);
+    if (DT != MF_F32 && NT > 1) return MF_WIDE_WAVES(DP);
     return (row_bytes <= 128 || (row_bytes <= 256 && NT == 1)) ? 2 : 1;
 }
 
@@ -456,26 +475,16 @@ constexpr int attn_waves_per_eu() {
 // workgroup (attn_mixed_kernel) sizes the arena for the larger, not for both.
 extern __shared__ __attribute__((aligned(16))) char attn_lds[];
 
-// Workgroup-shared prefill loop: tiles per LDS stage, and stage buffers (the
-// stage being computed plus the ones in flight) for 128-byte rows. Measured
-// on the C2 engine layer (and the prefill items alone, between events):
-// 2 x 4 tiles 48.8-49.0 us (35.4-35.8), 4 x 2 50.3 (36.3-36.5), 3 x 3
-// 49.1-49.4 (36.2-36.4), 3 x 2 49.6-50.1 (36.2-36.5), 3 x 4 55.4-55.6 (48 KB
-// of LDS: three workgroups per CU). More tiles in flight do not help: the
-// loop does not wait on memory.
-#ifndef MF_WIDE_TPS128
-#define MF_WIDE_TPS128 4
+// Workgroup-shared prefill loop (attn_wide_body): keys per LDS stage (two
+// stage buffers: the stage being computed and the one arriving).
+#ifndef MF_WIDE_KEYS
+#define MF_WIDE_KEYS(dp) ((dp) == 128 ? 32 : 64)
 #endif
-#ifndef MF_WIDE_NBUF128
-#define MF_WIDE_NBUF128 2
-#endif
-constexpr int wide_tps(int rb) { return rb == 128 ? MF_WIDE_TPS128 : 2; }
-constexpr int wide_nbuf(int rb) { return rb == 128 ? MF_WIDE_NBUF128 : 2; }
+constexpr int wide_keys(int dp) { return MF_WIDE_KEYS(dp); }
 template <int DT, int DP>
 constexpr int wide_lds_bytes() {
-    constexpr int rb = DP * (DT == MF_F32 ? 4 : 2);
     if constexpr (DT == MF_F32) return 0;  // the workgroup-shared loop is 16-bit only
-    else return wide_nbuf(rb) * wide_tps(rb) * 32 * rb + 16;
+    else return 2 * 2 * wide_keys(DP) * DP * 2;
 }
 template <int DP>
 constexpr int coop_lds_bytes() {
@@ -743,158 +752,6 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const int block) {
             load_tile(max(kt0, min(kt0 + i, pool_end - 1)), kR[i], vR[i], kt0 + i > pool_end - 1, none);
     }
 
-    // ---- workgroup-shared key loop, first part. Wide items whose workgroup
-    // shares one key range (the planner packs wide items that way, one column
-    // group per wave) stage each 16-key K/V tile in LDS for all four waves
-    // (the loop itself follows below). Its first stage needs only the item and
-    // the block table, so it is fetched here, before the row positions are
-    // waited for: the setup then costs the block table's round trip and the
-    // stage's, overlapped with the positions', instead of three in a row
-    // (the positions only trim how far the range is read; the first stage is
-    // bounded by the item's range instead). On a written-in-flight step the
-    // loop also takes the tiles holding new rows, reading each lane's key from
-    // the pool or from the new rows.
-    constexpr int RB = DP * ES;             // bytes of one key row
-    constexpr int NCH = RB / 16;            // 16-byte chunks per row
-    constexpr int STAGE = 32 * RB;          // K tile, then V tile
-    constexpr int NI = (STAGE + kWaves * 1024 - 1) / (kWaves * 1024);  // 16-byte loads per lane per tile
-    // Tiles per LDS stage: each barrier and each refill covers TPS
-    // tiles, so a refill has TPS tiles of compute to arrive in.
-    // Measured on the C2 prefill items (bf16, D 64): 1 tile 42.0 us,
-    // 2 tiles 40.3 us, 4 tiles 39.2 us. Four would take the D 32
-    // kernel past 128 registers (three waves per SIMD), so other row
-    // sizes use two.
-    constexpr int TPS = wide_tps(RB);
-    constexpr int NBUF = wide_nbuf(RB);
-    static_assert(NBUF >= 2 && NBUF <= 5 && (MF_WIDE_DIRECT_LDS || NBUF == 2), "stage buffers");
-    // this lane's 16 bytes of each tile: LDS byte base + lane*16 of
-    // piece (i*4 + wave) mod STAGE, and the matching pool offset inside
-    // the block (vector types rather than arrays keep them in registers)
-    typedef uint32_t offs_t __attribute__((ext_vector_type(NI)));
-    typedef uint32_t regs_t __attribute__((ext_vector_type(4 * NI * TPS)));
-    bool wg_shared = false;
-    if constexpr (FAST && DT != MF_F32 && NT > 1) {
-        if ((block + 1) * kWaves <= num_items) {
-            // The four items' (sequence, kv head, key range) are loaded
-            // together and compared without short-circuit: chained && made
-            // the compiler issue one load per comparison, each behind a full
-            // wait -- twelve round trips before the first K/V fetch, which
-            // beside a decode workgroup's streams took 12.7 us of a prefill
-            // workgroup's setup (4.0 us alone).
-            const int32_t* i0 = a.items + (int64_t)block * kWaves * MF_PLAN_ITEM_INTS;
-            int32_t key[kWaves][4];
-#pragma unroll
-            for (int w = 0; w < kWaves; ++w) {
-                const int32_t* iw = i0 + w * MF_PLAN_ITEM_INTS;
-                key[w][0] = iw[0];
-                key[w][1] = iw[1];
-                key[w][2] = iw[4];
-                key[w][3] = iw[5];
-            }
-            bool same = true;
-#pragma unroll
-            for (int w = 1; w < kWaves; ++w)
-                same = same & (key[w][0] == key[0][0]) & (key[w][1] == key[0][1]) & (key[w][2] == key[0][2]) &
-                       (key[w][3] == key[0][3]);
-            wg_shared = same;
-        }
-    }
-    const bool shared_inflight = TAIL && wg_shared;
-    offs_t src_off, key_of, piece_of;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const int base = ((i * kWaves + wave) * 1024) % STAGE;
-        const bool isv = base >= 16 * RB;
-        const int p2 = (isv ? base - 16 * RB : base) + lane * 16;
-        const int key = p2 / RB, slot = (p2 % RB) >> 4;
-        const int q = isv ? slot : (slot ^ (key & (NCH - 1)));
-        src_off[i] = (uint32_t)key * v_row_bytes + (uint32_t)q * 16;
-        key_of[i] = (uint32_t)key;
-        piece_of[i] = (uint32_t)q * 16;
-    }
-    // in-flight key k of this kv head: K row at ibase + k * irow_bytes,
-    // its V row iv_off bytes on (so the loop holds three numbers, not
-    // both tensors and their strides)
-    const char* ibase = a.new_k;
-    int64_t irow_bytes = 0, iv_off = 0;
-    if (shared_inflight) {
-        irow_bytes = a.n_sr * ES;
-        ibase = a.new_k + ((int64_t)(row0 - pool_len) * a.n_sr + (int64_t)h * a.n_sh) * ES;
-        iv_off = a.new_v - a.new_k;
-    }
-    // Tiles the fetches clamp to: the item's range for the first stage, the
-    // workgroup's last read tile once the positions are in.
-    int fetch_end = kt1;
-    // Loads are unconditional (a wave without a piece of a small tile
-    // re-reads another wave's piece and does not store it; tiles past
-    // the range re-read the last one): a conditional load would make
-    // every later wait drain all loads.
-    auto fetch = [&](int t0, regs_t& r) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < TPS; ++u) {
-            const int t = min(t0 + u, fetch_end - 1);
-            const int phys = tbl_at(t - kt0);
-            const int64_t boff = ((int64_t)phys * a.p_sb + (int64_t)h * a.p_sh) * ES;
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int base = ((i * kWaves + wave) * 1024) % STAGE;
-                const bool isv = base >= 16 * RB;
-                const char* src = (isv ? a.v_pool : a.k_pool) + boff + src_off[i];
-                if (shared_inflight) {
-                    // this lane's key is a new row of the sequence
-                    // (clamped to its last row past the context; those
-                    // keys are masked and their V cleared)
-                    const int key = t * 16 + (int)key_of[i];
-                    const char* isrc = ibase + (isv ? iv_off : 0) +
-                                       (int64_t)min(key, kv_len - 1) * irow_bytes + piece_of[i];
-                    src = key >= pool_len ? isrc : src;
-                }
-                const uint4 v = *(const uint4*)src;
-                const int w = 4 * (u * NI + i);
-                r[w] = v.x;
-                r[w + 1] = v.y;
-                r[w + 2] = v.z;
-                r[w + 3] = v.w;
-            }
-        }
-    };
-    // The same stage straight into LDS buffer `buf` (direct form): each wave
-    // writes its 1 KB pieces of each tile; a wave without a piece of a small
-    // tile loads nothing.
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)attn_lds;
-    auto dfetch = [&](int t0, int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < TPS; ++u) {
-            const int t = min(t0 + u, fetch_end - 1);
-            const int phys = tbl_at(t - kt0);
-            const int64_t boff = ((int64_t)phys * a.p_sb + (int64_t)h * a.p_sh) * ES;
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int base = (i * kWaves + wave) * 1024;
-                if (base >= STAGE) continue;
-                const bool isv = base >= 16 * RB;
-                const char* src = (isv ? a.v_pool : a.k_pool) + boff + src_off[i];
-                if (shared_inflight) {
-                    const int key = t * 16 + (int)key_of[i];
-                    const char* isrc = ibase + (isv ? iv_off : 0) +
-                                       (int64_t)min(key, kv_len - 1) * irow_bytes + piece_of[i];
-                    src = key >= pool_len ? isrc : src;
-                }
-                ld_lds16(src, lds_base + (uint32_t)((buf * TPS + u) * STAGE + base));
-            }
-        }
-    };
-    regs_t rs;
-    if constexpr (FAST && DT != MF_F32 && NT > 1) {
-        if (wg_shared) {
-            if constexpr (MF_WIDE_PRIO > 0) __builtin_amdgcn_s_setprio(MF_WIDE_PRIO);
-            if (kt1 > kt0) {
-                if constexpr (MF_WIDE_DIRECT_LDS) dfetch(kt0, 0);
-                else fetch(kt0, rs);
-            }
-        }
-    }
-
     int maxpos = -1;
     int minpos = INT_MAX;  // over the item's real columns
 #pragma unroll
@@ -941,7 +798,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const int block) {
     // candidates follow through the general per-key loads.
     int fast_end = kt_end;
     if constexpr (FAST) {
-        if (inflight && !shared_inflight) fast_end = max(kt0, min(kt_end, pool_len >> 4));
+        if (inflight) fast_end = max(kt0, min(kt_end, pool_len >> 4));
     }
     // Per-tile work is branch-free apart from wave-uniform decisions: every
     // column tile's MFMAs run (tiles past nct hold zero queries and are never
@@ -1079,138 +936,12 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const int block) {
     };
 
     // ---- key loops. Single-column-tile items (decode, verify) stream their
-    // own tiles through the NB-buffer register ring below; wide items either
-    // share each tile through LDS (next) or, pooled four to a workgroup with
-    // unrelated items, stream their own tiles through two buffers. Every
+    // own tiles through the NB-buffer register ring below; wide items pooled
+    // four to a workgroup with unrelated items stream theirs through two
+    // buffers (attn_wide_body runs the ones that share a key range). Every
     // prefetch is unconditional (past the end it is a dummy or a clamped
     // re-read) because a conditional load makes the compiler drain every
     // outstanding load at the join and serialises the pipeline.
-    // ---- workgroup-shared key loop (16-bit wide items on the fast path).
-    // When the workgroup's four items cover one (sequence, kv head, key
-    // range) -- the planner packs wide items that way, one column group per
-    // wave -- every 16-key K/V tile is fetched once for the workgroup (a
-    // quarter per wave, 16 bytes per lane) and staged in LDS, and each wave
-    // reads its MFMA fragments from LDS. That takes the four-fold re-reads of
-    // each tile off the texture path, which is what limits the per-wave loop
-    // on prefill. Tiles move in stages of TPS: loads run one stage ahead in
-    // registers; LDS holds two stages (a stage is written after the barrier
-    // that retires the previous reads of its buffer). Each K row's 16-byte
-    // chunks are stored xor-swizzled by key, so the fragment reads (16 keys x
-    // one chunk) hit distinct banks; V rows are read 16 lanes to a row,
-    // conflict-free. One barrier per stage.
-    if constexpr (FAST && DT != MF_F32 && NT > 1) {
-        if (wg_shared) {
-            static_assert(wide_lds_bytes<DT, DP>() == NBUF * TPS * STAGE + 16, "LDS arena layout");
-            char* smem = attn_lds;
-            int* s_end = reinterpret_cast<int*>(attn_lds + NBUF * TPS * STAGE);
-            if (lane == 0) s_end[wave] = fast_end;
-            __syncthreads();
-            const int wg_end = __builtin_amdgcn_readfirstlane(
-                max(max(s_end[0], s_end[1]), max(s_end[2], s_end[3])));
-            const int n = wg_end - kt0;
-            fetch_end = wg_end;
-            auto stash = [&](const regs_t& r, int buf) __attribute__((always_inline)) {
-#pragma unroll
-                for (int u = 0; u < TPS; ++u) {
-#pragma unroll
-                    for (int i = 0; i < NI; ++i) {
-                        const int base = (i * kWaves + wave) * 1024;
-                        const int w = 4 * (u * NI + i);
-                        if (base < STAGE)
-                            *(uint4*)(smem + (buf * TPS + u) * STAGE + base + lane * 16) =
-                                make_uint4(r[w], r[w + 1], r[w + 2], r[w + 3]);
-                    }
-                }
-            };
-            auto sync = [&]() {
-                // this wave's LDS reads and writes are done, then all waves'
-                __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (7 << 4) | (0 << 8));  // lgkmcnt(0)
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
-            };
-            auto wait_stages = [&](int pending) {
-                // this wave's direct loads done, but for the last `pending` stages
-                if (pending <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                else if (pending == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(TPS * NI) : "memory");
-                else if (pending == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * TPS * NI) : "memory");
-                else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * TPS * NI) : "memory");
-            };
-            if (n > 0 && MF_WIDE_DIRECT_LDS) {
-                // NBUF buffers: stage u is computed while stages u+1 ..
-                // u+NBUF-1 arrive; after the barrier that ends stage u (every
-                // wave is done reading its buffer, and has waited for its own
-                // pieces of stage u+1), stage u+NBUF is issued into it.
-                const int nst = (n + TPS - 1) / TPS;
-                // the first stage went out with the setup loads
-                for (int s = 1; s < NBUF; ++s)
-                    if (s < nst) dfetch(kt0 + s * TPS, s);
-                wait_stages(min(NBUF - 1, nst - 1));
-                sync();
-                int buf = 0;
-                for (int u = 0; u < nst; ++u) {
-                    // fragments of staged tile v (K rows swizzled, V rows plain)
-                    auto frags = [&](int v, uint4 (&kf)[NL], uint32_t (&vf)[4][VWD]) {
-                        const char* stg = smem + (buf * TPS + v) * STAGE;
-#pragma unroll
-                        for (int c = 0; c < NL; ++c)
-                            kf[c] = *(const uint4*)(stg + j * RB + (((c * 4 + g) ^ (j & (NCH - 1))) << 4));
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) ld_words<VB>(stg + 16 * RB + (4 * g + r) * RB + j * VB, vf[r]);
-                    };
-#pragma unroll
-                    for (int v = 0; v < TPS; ++v) {
-                        const int t = kt0 + u * TPS + v;
-                        if (t < fast_end) {
-                            uint4 kf[NL];
-                            uint32_t vf[4][VWD];
-                            frags(v, kf, vf);
-                            process(t, kf, vf);
-                        }
-                    }
-                    wait_stages(min(NBUF - 2, nst - 2 - u));
-                    sync();
-                    if (u + NBUF < nst) dfetch(kt0 + (u + NBUF) * TPS, buf);
-                    buf = buf + 1 == NBUF ? 0 : buf + 1;
-                }
-            } else if (n > 0) {
-                // Register form (two LDS buffers): one register set in
-                // flight; stage u+1 (TPS tiles) arrives during stage u's
-                // compute, is stored to the other LDS buffer, and the set is
-                // refilled with stage u+2.
-                const int nst = (n + TPS - 1) / TPS;
-                stash(rs, 0);  // the first stage, fetched with the setup loads
-                fetch(kt0 + TPS, rs);
-                sync();
-                for (int u = 0; u < nst; ++u) {
-                    // fragments of staged tile v (K rows swizzled, V rows plain)
-                    auto frags = [&](int v, uint4 (&kf)[NL], uint32_t (&vf)[4][VWD]) {
-                        const char* stg = smem + ((u & 1) * TPS + v) * STAGE;
-#pragma unroll
-                        for (int c = 0; c < NL; ++c)
-                            kf[c] = *(const uint4*)(stg + j * RB + (((c * 4 + g) ^ (j & (NCH - 1))) << 4));
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) ld_words<VB>(stg + 16 * RB + (4 * g + r) * RB + j * VB, vf[r]);
-                    };
-#pragma unroll
-                    for (int v = 0; v < TPS; ++v) {
-                        const int t = kt0 + u * TPS + v;
-                        if (t < fast_end) {
-                            uint4 kf[NL];
-                            uint32_t vf[4][VWD];
-                            frags(v, kf, vf);
-                            process(t, kf, vf);
-                        }
-                    }
-                    if (u + 1 < nst) {
-                        stash(rs, (u + 1) & 1);
-                        fetch(kt0 + (u + 2) * TPS, rs);
-                    }
-                    sync();
-                }
-            }
-        }
-    }
     // The first tile past the pipelined range (a verify pass's boundary or
     // candidate tile) is fetched before the loop, so its per-key loads
     // overlap the pool tiles instead of following them.
@@ -1219,7 +950,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const int block) {
     if constexpr (FAST && NT == 1) {
         if (fast_end < kt_end) load_general(fast_end, kT, vT);
     }
-    if (kt0 < fast_end && !wg_shared) {
+    if (kt0 < fast_end) {
         // Ring of NB register buffers: each step issues the tile NB-1 ahead
         // into the slot freed last and processes the oldest. The loop runs
         // whole rounds of NB steps and the last n % NB tiles (already in
@@ -1401,24 +1132,411 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const int block) {
         }
     }
 
-    // ---- fused split-K merge: the last partition of a group to arrive merges
-    // the group. Release the partials (agent-scope fence: the L2s of the XCDs
-    // are not coherent with each other), count the arrival, and on the last
-    // arrival acquire everyone else's partials and reset the counter for the
-    // next call. Every wave runs to the end; nothing waits on another wave.
-    if (pslot >= 0 && a.counters != nullptr) {
-        const int m0 = iv1.w;
-        __threadfence();
-        int prev = 0;
-        if (lane == 0) prev = atomicAdd(a.counters + m0, 1);
-        prev = __shfl(prev, 0, 64);
-        const int32_t* mg0 = a.merges + (int64_t)m0 * MF_PLAN_MERGE_INTS;
-        if (prev == mg0[3] - 1) {
-            __threadfence();
-            if (lane == 0) a.counters[m0] = 0;
-            for (int o = 0; o < nct; ++o) merge_tile<DT, DP>(a, mg0 + o * MF_PLAN_MERGE_INTS, g, j);
+    if (pslot >= 0) arrive_and_merge<DT, DP>(a, iv1.w, nct, lane);
+}
+
+// ------------------------------------------------- workgroup-shared wide items
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+// S^T / O^T block: 32 rows x 32 columns, contraction over 16 elements (8 per
+// lane half).
+template <int DT>
+__device__ __forceinline__ f32x16 mfma32(uint4 a, uint4 b, f32x16 c) {
+    if constexpr (DT == MF_BF16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                       0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c,
+                                                      0, 0, 0);
+}
+
+// 4 keys x 16 head_dim elements per 16-lane group, transposed on the way out
+// of LDS: lane i of the group gets element i of the four rows.
+__device__ __forceinline__ uint2 ld_tr16(const char* lds) {
+    typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)lds));
+}
+
+// ld_lds16 from a wave-uniform base and a 32-bit lane offset: no vector
+// address arithmetic per load. The five wait states cover a base that a vector
+// instruction (v_readfirstlane) wrote just before, which the compiler cannot
+// see to do inside the assembly, and the m0 write's one.
+__device__ __forceinline__ void ld_lds16_base(const char* base_, uint32_t lane_off, uint32_t lds_addr) {
+    const uint64_t u = (uint64_t)(uintptr_t)base_;
+    const uint64_t base = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)u) |
+                          ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(u >> 32)) << 32);
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds_addr), "v"(lane_off), "s"(base) : "memory");
+}
+
+// A workgroup whose four wide items are column groups of one (sequence, kv
+// head, key range): each wave owns 32 columns, and every K/V row of the range
+// is staged in LDS once for the four waves.
+//
+// Per 32 keys the wave forms S^T = K Q^T and O^T += V^T P^T as 32x32x16 MFMA
+// blocks (the full-rate shape: 1.85 PFLOP/s over the chip on this card against
+// 1.17 for 16x16x32 and half that for 16x16x16). S^T leaves lane (half hf,
+// column c) with keys 8b + 4hf + r of its column; P^T's B operand takes those
+// registers as they are, and V^T's A operand is read in the same key order by
+// the transposing LDS read, so neither P nor V moves between lanes.
+//
+// Stages of 64 keys go from global memory straight into LDS (two buffers, one
+// barrier per stage). Each wave loads the same few 1 KB pieces of every
+// 16-key block, so a piece is one scalar base plus a lane offset that never
+// changes: new rows of a written-in-flight step are just another base and
+// offset. K rows are xor-swizzled by key in 16-byte chunks (32 keys x one
+// chunk read conflict-free), V rows by key mod 4 in pairs of 32-byte granules
+// (the transposing read's four rows x 64 bytes hit distinct banks): the
+// conflict counter reads zero.
+//
+// Measured on MI355X against the 16x16 loop this replaces (one layer, KV write
+// and merge included): two chunks of 2048 rows after up to 6144 keys, 40/8
+// heads x 128, 333 GFLOP: 817 -> 388 us (860 TFLOP/s); 16 prompts of up to 1024
+// tokens, 15/5 heads x 64: 32.9 -> 29.1 us. What bounds it: MFMA is busy a third
+// of the time and the VALU (exponentials, maxima, packing) as long, in turn
+// rather than together -- timing copies without the exponentials, the PV
+// products or the LDS reads each gained 10-25%, none more. So waves per SIMD
+// count: at 256-byte rows 32-key stages leave room for three (168 registers,
+// 32 KB of LDS a workgroup), 373 us against 403 with two and 64-key stages;
+// two score chains at a time took 430 against 436. Scalar registers count too:
+// a base computed for every load apart, with a branch each, took 630 us.
+template <int DT, int DP, bool TAIL>
+__device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int block) {
+    constexpr int RB = DP * 2;       // bytes of one key row
+    constexpr int NCH = RB / 16;     // 16-byte chunks per row
+    constexpr int KEYS = wide_keys(DP), TS = KEYS / 16;  // keys and 16-key blocks per stage
+    constexpr int RPB = 256 / RB;    // rows per 256 bytes (all LDS banks once)
+    constexpr int NQ = DP / 16;      // MFMA steps of S^T
+    constexpr int ND = DP / 32;      // 32-row blocks of O^T
+    constexpr int PK = RB / 64;      // 1 KB pieces of 16 K rows (V: as many)
+    constexpr int NLD = TS * 2 * PK / 4;  // pieces per wave and stage
+    constexpr int NOFF = DP == 128 ? 2 : 1;  // a wave's distinct pieces of a block
+    constexpr int HALF = KEYS * RB;     // K rows of a stage, then its V rows
+    constexpr int STG = 2 * HALF;
+    static_assert(DT != MF_F32 && RPB >= 1 && wide_lds_bytes<DT, DP>() == 2 * STG, "stage layout");
+    constexpr float kNegInf = -__builtin_huge_valf();
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int hf = lane >> 5;
+    const char *k_pool = a.k_pool, *v_pool = a.v_pool, *new_k = a.new_k, *new_v = a.new_v;
+    const int32_t* items = a.items + (int64_t)block * kWaves * MF_PLAN_ITEM_INTS;
+    const int32_t* it = items + wave * MF_PLAN_ITEM_INTS;
+    const int s = it[0], h = it[1], c0 = it[2], nct = it[3], kt0 = it[4], kt1 = it[5], pslot = it[6], m0 = it[7];
+    const int row0 = it[8], nrows = it[9], kv_len = it[10];
+    const bool inflight = TAIL || a.pool_lens != nullptr;
+    const int pool_len = TAIL ? kv_len - nrows : (a.pool_lens != nullptr ? a.pool_lens[s] : kv_len);
+
+    // block-table entries of the 64 tiles from tbl_base (one per lane), and of
+    // the 64 after them
+    const int32_t* trow = a.block_tables + (int64_t)s * a.bt_stride;
+    const int tbl_end = inflight ? min(kt1, (pool_len + 15) >> 4) : kt1;
+    const int tbl_last = max(tbl_end - 1, 0);  // tiles past it are new rows: never read through the table
+    int tbl_base = kt0;
+    int tbl = trow[min(kt0 + lane, tbl_last)], tbl_next = trow[min(kt0 + 64 + lane, tbl_last)];
+    auto tbl_at = [&](int t) -> int { return __builtin_amdgcn_readlane(tbl, t - tbl_base); };  // wave-uniform t
+
+    // ---- this lane's column: position and query (padding columns read
+    // row0's and are never stored)
+    const int ct = (lane & 31) >> 4, j = lane & 15;
+    const int cidx = c0 * 16 + (lane & 31);
+    const bool valid = ct < nct && cidx < nrows * a.G;
+    const int crow = valid ? cidx / a.G : 0;
+    const int qhead = h * a.G + (valid ? cidx - crow * a.G : 0);
+    int prow = row0 + crow;
+    if (a.row_map) prow = a.row_map[prow];
+    const int pos = reinterpret_cast<const int32_t*>(a.positions)[2 * (int64_t)prow];
+    const int qpos = valid ? pos : -1;
+    // the positions of the workgroup's other columns (two per lane): how far
+    // its stages run, without an exchange between the waves
+    int wpos = -1;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int32_t* iw = items + (2 * k + hf) * MF_PLAN_ITEM_INTS;
+        const int c = iw[2] * 16 + (lane & 31);
+        const bool v = ct < iw[3] && c < nrows * a.G;
+        int r = row0 + (v ? c / a.G : 0);
+        if (a.row_map) r = a.row_map[r];
+        const int x = reinterpret_cast<const int32_t*>(a.positions)[2 * (int64_t)r];
+        wpos = max(wpos, v ? x : -1);
+    }
+    uint4 qf[NQ];
+#pragma unroll
+    for (int c = 0; c < NQ; ++c) {
+        const uint4 v = *(const uint4*)(a.q + ((int64_t)prow * a.q_sr + (int64_t)qhead * a.q_sh + c * 16 + hf * 8) * 2);
+        qf[c] = make_uint4(v.x ^ a.q_sign, v.y ^ a.q_sign, v.z ^ a.q_sign, v.w ^ a.q_sign);
+    }
+
+    // ---- stages
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)attn_lds;
+    uint32_t off[NOFF], ioff[NOFF];  // this lane's 16 bytes inside a 16-key block: pool rows, new rows
+#pragma unroll
+    for (int n = 0; n < NOFF; ++n) {
+        const int p = (wave + 4 * n) % (2 * PK);
+        const bool isv = p >= PK;
+        const int k16 = (isv ? p - PK : p) * (1024 / RB) + lane * 16 / RB;
+        const int swz = isv ? ((k16 & 3) / RPB) << 2 : (k16 / RPB) & (NCH - 1);
+        const uint32_t piece = (uint32_t)(((lane & (NCH - 1)) ^ swz) << 4);
+        off[n] = (uint32_t)(k16 * a.p_ss * 2) + piece;
+        ioff[n] = (uint32_t)(k16 * a.n_sr * 2) + piece;
+    }
+    const int64_t blk_bytes = a.p_sb * 2;
+    const char* kp_h = k_pool + (int64_t)h * a.p_sh * 2;  // this kv head's rows
+    const char* nk_h = new_k + ((int64_t)(row0 - pool_len) * a.n_sr + (int64_t)h * a.n_sh) * 2;
+    const int64_t v_delta = v_pool - k_pool, nv_delta = new_v - new_k;
+    const int64_t tile_bytes = 16 * a.n_sr * 2;
+    // tiles the fetches clamp to: the item's range for the first stage, the
+    // workgroup's last read tile once the positions are in
+    int fetch_end = kt1;
+    auto fetch = [&](int u, int buf) __attribute__((always_inline)) {
+        const int t0 = kt0 + TS * u;
+        if (t0 - tbl_base >= 64) {
+            tbl_base += 64;
+            tbl = tbl_next;
+            tbl_next = trow[min(tbl_base + 64 + lane, tbl_last)];
+        }
+        const uint32_t dst0 = lds_base + (uint32_t)(buf * STG);
+        const int key1 = (t0 + TS) * 16;
+        const bool whole = t0 + TS <= fetch_end;
+        // A stage wholly in the pool or wholly of new rows takes a scalar base
+        // per block; the boundary stage, the range's last one, and rows behind
+        // a row map take the general form below.
+        const bool in_pool = whole & (!inflight | (key1 <= pool_len));
+        const bool in_new = whole & inflight & (t0 * 16 >= pool_len) & (key1 <= kv_len) & (a.row_map == nullptr);
+        auto piece = [&](int i, const char* block_base, int64_t to_v, uint32_t lane_off) {
+            const int p = (wave + 4 * i) % (2 * PK), b = (wave + 4 * i) / (2 * PK);
+            const bool isv = p >= PK;
+            ld_lds16_base(block_base + (isv ? to_v : 0), lane_off,
+                          dst0 + (uint32_t)(b * 16 * RB + (isv ? HALF + (p - PK) * 1024 : p * 1024)));
+        };
+        if (in_pool) {
+#pragma unroll
+            for (int i = 0; i < NLD; ++i)
+                piece(i, kp_h + (int64_t)tbl_at(t0 + (wave + 4 * i) / (2 * PK)) * blk_bytes, v_delta, off[i % NOFF]);
+        } else if (in_new) {
+#pragma unroll
+            for (int i = 0; i < NLD; ++i)
+                piece(i, nk_h + (t0 + (wave + 4 * i) / (2 * PK)) * tile_bytes, nv_delta, ioff[i % NOFF]);
+        } else {
+#pragma unroll 1
+            for (int i = 0; i < NLD; ++i) {
+                const int x = wave + 4 * i;
+                const int b = x / (2 * PK), p = x % (2 * PK);
+                const bool isv = p >= PK;
+                const int t = min(t0 + b, fetch_end - 1);
+                const uint32_t dst = dst0 + (uint32_t)(b * 16 * RB + (isv ? HALF + (p - PK) * 1024 : p * 1024));
+                const int k16 = (isv ? p - PK : p) * (1024 / RB) + lane * 16 / RB;
+                const int swz = isv ? ((k16 & 3) / RPB) << 2 : (k16 / RPB) & (NCH - 1);
+                const int piece = ((lane & (NCH - 1)) ^ swz) << 4;
+                // In a block of the pool every slot exists; a new row past the
+                // context reads the last one. Either is masked, and its V row
+                // cleared.
+                const int key = inflight ? min(t * 16 + k16, kv_len - 1) : t * 16 + k16;
+                const char* src;
+                if (!inflight || key < pool_len) {
+                    const int64_t blk = tbl_at(t);
+                    src = k_pool + (isv ? v_delta : 0) + (blk * a.p_sb + (int64_t)k16 * a.p_ss + (int64_t)h * a.p_sh) * 2;
+                } else {
+                    int nr = row0 + key - pool_len;
+                    if (a.row_map) nr = a.row_map[nr];
+                    src = new_k + (isv ? nv_delta : 0) + ((int64_t)nr * a.n_sr + (int64_t)h * a.n_sh) * 2;
+                }
+                ld_lds16(src + piece, dst);
+            }
+        }
+    };
+    if constexpr (MF_WIDE_PRIO > 0) __builtin_amdgcn_s_setprio(MF_WIDE_PRIO);
+    if (kt1 > kt0) fetch(0, 0);
+
+    // ---- the columns' causal limits; tiles past the workgroup's last visible
+    // key are not read
+    const int end_key = min(kv_len, kt1 * 16);
+    const int lim = qpos >= 0 ? min(qpos, end_key - 1) : -1;  // last key the column may see here
+    int maxlim = lim, minlim = valid ? lim : INT_MAX, wglim = min(wpos, end_key - 1);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        maxlim = max(maxlim, __shfl_xor(maxlim, o, 64));
+        minlim = min(minlim, __shfl_xor(minlim, o, 64));
+        wglim = max(wglim, __shfl_xor(wglim, o, 64));
+    }
+    maxlim = __builtin_amdgcn_readfirstlane(maxlim);
+    minlim = __builtin_amdgcn_readfirstlane(minlim);
+    wglim = __builtin_amdgcn_readfirstlane(wglim);
+    auto sync = [&]() {
+        // this wave's LDS reads and writes are done, then all waves'
+        __builtin_amdgcn_s_waitcnt((15) | (3 << 14) | (7 << 4) | (0 << 8));  // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    const int wg_end = wglim < kt0 * 16 ? kt0 : (wglim >> 4) + 1;
+    fetch_end = wg_end;
+    const int nst = (wg_end - kt0 + TS - 1) / TS;
+
+    float m = kMinM, l = 0.f;
+    float thr = (kMinM + kLazyLog2) * a.inv_scale_log2;
+    f32x16 acc[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] = 0.f;
+
+    // lane addresses inside a stage: K rows (key lane & 31), V rows (key 4hf +
+    // (lane & 15) / 4 of each group of 8)
+    uint32_t kaddr[NQ], vaddr[ND];
+#pragma unroll
+    for (int c = 0; c < NQ; ++c)
+        kaddr[c] = (uint32_t)((lane & 31) * RB + (((2 * c + hf) ^ ((j / RPB) & (NCH - 1))) << 4));
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+        vaddr[d] = (uint32_t)(HALF + (4 * hf + (j >> 2)) * RB +
+                              (((4 * d + 2 * ct + ((j & 3) >> 1)) ^ (((j >> 2) / RPB) << 2)) << 4) + 8 * (j & 1));
+
+    auto tile = [&](const char* stg, int key0) __attribute__((always_inline)) {
+        f32x16 st;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st[i] = 0.f;
+#pragma unroll
+        for (int c = 0; c < NQ; ++c) st = mfma32<DT>(*(const uint4*)(stg + kaddr[c]), qf[c], st);
+        if (key0 + 31 > minlim) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                st[i] = key0 + 8 * (i >> 2) + 4 * hf + (i & 3) <= lim ? st[i] : kNegInf;
+        }
+        // lazy rescale, as in attn_body; a column's keys lie in two lanes
+        float lmax = st[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) lmax = fmax_prop(lmax, st[i]);
+        if (__builtin_amdgcn_ballot_w64(lmax > thr) != 0) {
+            auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(lmax), __float_as_uint(lmax), false, false);
+            const float cm = fmax_prop(__uint_as_float(r[0]), __uint_as_float(r[1]));
+            const float mn = fmaxf(m, cm * a.scale_log2);
+            const float alpha = __builtin_amdgcn_exp2f(m - mn);
+            l *= alpha;
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[d][i] *= alpha;
+            m = mn;
+            thr = (mn + kLazyLog2) * a.inv_scale_log2;
+        }
+        uint32_t pw[8];
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * i], a.scale_log2, -m));
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * i + 1], a.scale_log2, -m));
+            sum += p0 + p1;
+            if constexpr (DT == MF_BF16)
+                pw[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){p0, p1}, bf16x2));
+            else
+                pw[i] = f32_to_bits<DT>(p0) | (f32_to_bits<DT>(p1) << 16);
+        }
+        l += sum;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const uint4 pf = make_uint4(pw[4 * k], pw[4 * k + 1], pw[4 * k + 2], pw[4 * k + 3]);
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                const uint2 v0 = ld_tr16(stg + vaddr[d] + (16 * k) * RB);
+                const uint2 v1 = ld_tr16(stg + vaddr[d] + (16 * k + 8) * RB);
+                acc[d] = mfma32<DT>(make_uint4(v0.x, v0.y, v1.x, v1.y), pf, acc[d]);
+            }
+        }
+    };
+
+    if (nst > 0) {
+        if (nst > 1) fetch(1, 1);
+        const int live_end = min(kv_len, wg_end * 16);  // rows past it may hold anything, NaN included
+        if (nst > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NLD) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        sync();
+        for (int u = 0; u < nst; ++u) {
+            char* stg = attn_lds + (u & 1) * STG;
+            const int key0 = (kt0 + TS * u) * 16;
+            if (key0 + KEYS > live_end) {
+                // the last stage: p is 0 for its rows past the context, and 0 * NaN is NaN
+                const int first = live_end - key0;
+                for (int x = first * NCH + (int)threadIdx.x; x < KEYS * NCH; x += 256)
+                    *(uint4*)(stg + HALF + x * 16) = make_uint4(0, 0, 0, 0);
+                sync();
+            }
+#pragma unroll
+            for (int v = 0; v < KEYS / 32; ++v)
+                if (key0 + 32 * v <= maxlim) tile(stg + v * 32 * RB, key0 + 32 * v);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            sync();
+            if (u + 2 < nst) fetch(u + 2, u & 1);
+        }
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first stage still lands in this workgroup's LDS
+    }
+
+    // ---- finish: lane (hf, column) holds head_dim elements 32d + 8b + 4hf ..
+    // + 3; the halves trade blocks so that each lane stores 16 bytes
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    const float lt = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const float inv = lt > 0.f ? 1.f / lt : 0.f;
+    char* dst = nullptr;
+    if (qpos >= 0)
+        dst = pslot < 0 ? a.out + ((int64_t)prow * a.o_sr + (int64_t)qhead * a.o_sh) * 2
+                        : partial_out<DT>(a, pslot + ct, j, 0);
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int b = 0; b < 4; b += 2) {
+            uint32_t w[2][2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    w[e][k] = f32_to_bits<DT>(acc[d][4 * (b + e) + 2 * k] * inv) |
+                              (f32_to_bits<DT>(acc[d][4 * (b + e) + 2 * k + 1] * inv) << 16);
+            auto x = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
+            auto y = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
+            if (qpos >= 0) *(uint4*)(dst + (32 * d + 8 * (b + hf)) * 2) = make_uint4(x[0], y[0], x[1], y[1]);
+        }
+    if (pslot >= 0) {
+        if (qpos >= 0 && hf == 0) {
+            float* ml = partial_ml(a, pslot + ct);
+            ml[j] = m;
+            ml[16 + j] = lt;
+        }
+        arrive_and_merge<DT, DP>(a, m0, nct, lane);
+    }
+}
+
+// One workgroup of a launch's items. 16-bit wide items share their key range
+// through LDS: the planner gives every such workgroup one (sequence, kv head,
+// key range); one whose items differ runs them wave by wave. The four items'
+// fields are loaded together and compared without short-circuit: chained &&
+// made the compiler issue one load per comparison, each behind a full wait,
+// which beside a decode workgroup's streams took 12.7 us of a prefill
+// workgroup's setup (4.0 us alone).
+template <int DT, int DP, int NT, bool FAST, bool TAIL = false>
+__device__ __forceinline__ void attn_block(const AttnArgs& a, const int block) {
+    if constexpr (FAST && DT != MF_F32 && NT > 1) {
+        const int num_items = a.dev_count ? *a.dev_count : a.num_items;
+        const int32_t* i0 = a.items + (int64_t)block * kWaves * MF_PLAN_ITEM_INTS;
+        int32_t key[kWaves][4];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const int32_t* iw = i0 + w * MF_PLAN_ITEM_INTS;
+            key[w][0] = iw[0];
+            key[w][1] = iw[1];
+            key[w][2] = iw[4];
+            key[w][3] = iw[5];
+        }
+        bool same = (block + 1) * kWaves <= num_items;
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w)
+            same = same & (key[w][0] == key[0][0]) & (key[w][1] == key[0][1]) & (key[w][2] == key[0][2]) &
+                   (key[w][3] == key[0][3]);
+        if (same) {
+            attn_wide_body<DT, DP, TAIL>(a, block);
+            return;
         }
     }
+    attn_body<DT, DP, NT, FAST, TAIL>(a, block);
 }
 
 // The item list comes as a separate first argument, which the build has the
@@ -1433,9 +1551,9 @@ void attn_kernel(const int32_t* items, AttnArgs a) {
         // layer against 55.7 with them last)
         const int b = blockIdx.x;
         if (b < a.w_blocks) write_new_rows<DT>(a, b);
-        else attn_body<DT, DP, NT, FAST, true>(a, b - a.w_blocks);
+        else attn_block<DT, DP, NT, FAST, true>(a, b - a.w_blocks);
     } else {
-        attn_body<DT, DP, NT, FAST>(a, blockIdx.x);
+        attn_block<DT, DP, NT, FAST>(a, blockIdx.x);
     }
 }
 
@@ -1491,7 +1609,7 @@ void attn_mixed_kernel(AttnArgs narrow, AttnArgs wide, int wide_blocks) {
         narrow_start_delay();
         attn_body<DT, DP, 1, true>(narrow, b);
     } else {
-        attn_body<DT, DP, NTW, true>(wide, b - narrow_blocks);
+        attn_block<DT, DP, NTW, true>(wide, b - narrow_blocks);
     }
 }
 
@@ -1514,7 +1632,7 @@ void attn_mixed_tail_kernel(AttnArgs a, const int32_t* wide_items, int wide_num_
         w.items = wide_items;
         w.num_items = wide_num_items;
         w.dev_count = wide_dev_count;
-        attn_body<DT, DP, NTW, true, true>(w, b - narrow_blocks);
+        attn_block<DT, DP, NTW, true, true>(w, b - narrow_blocks);
     }
 }
 
@@ -1969,10 +2087,11 @@ inline int part_dstride_for(int head_dim) { return head_dim < 32 ? 32 : head_dim
 }  // namespace
 }  // namespace mf
 
-extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
-                                 int num_q_heads, int num_kv_heads, int head_dim, int dtype,
-                                 int partition_tiles, int32_t* items, int64_t items_capacity,
-                                 int32_t* merges, int64_t merges_capacity, int64_t* counts) {
+namespace {
+// The planner of mf_attention_plan (num_cus 0) and mf_attention_plan_device.
+int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens, int num_q_heads,
+                   int num_kv_heads, int head_dim, int dtype, int partition_tiles, int num_cus, int32_t* items,
+                   int64_t items_capacity, int32_t* merges, int64_t merges_capacity, int64_t* counts) {
     if (num_seqs < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || !counts)
         return MF_ERR_ARG;
     if (num_q_heads % num_kv_heads) return MF_ERR_ARG;
@@ -2153,12 +2272,25 @@ extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const 
     // to 37.9 us). The XCD queues below take a (sequence, kv head)'s quads
     // as one run: the launch fetches 1.09x its algorithmic reads, against
     // 1.65x with each (quad, kv head) dealt alone (0.3 us faster).
-    constexpr int kPlanCUs = 256;  // compute units of an MI355X
+    const int kPlanCUs = num_cus > 0 ? num_cus : 256;  // an MI355X has 256 compute units
+    // A plan made for a device cuts every wide sequence by quads -- also one of
+    // fewer than four column groups, whose quad has idle waves but whose tiles
+    // are shared -- and a shared workgroup's range may be any length (its block
+    // table is read 64 tiles at a time). At 128-byte rows and less, a plan of
+    // wide items only does so where the general ranges come out shorter than 32
+    // tiles (PW), and a workgroup's set-up costs more than its tiles: 15/5 heads
+    // x 64, device against general ranges, us: 1024 fresh rows (8 tiles) 18.1
+    // against 23.9, 8 prompts of up to 300 (4) 14.2 / 18.9, 256 rows after 6144
+    // keys (19) 24.3 / 27.7, but 4 chunks of 512 after up to 2048 (32) 25.6 /
+    // 28.6 and 16 prompts of up to 1024 (64) 30 / 32. At 256-byte rows it always
+    // does: 2 chunks of 2048 after 6144 keys 370 against 428 (10,240 merges).
+    const bool device = num_cus > 0 && partition_tiles <= 0 && WT > 1 && dtype != MF_F32 && head_dim == DP &&
+                        (mixed || DP >= 128 || PW < 32);
     auto quads = [&](int s) -> int {  // column quads of s, 0 if s is not a shared wide sequence
         const int nct = col_tiles(s);
-        if (!mixed || !nct || nct == 1 || WT == 1) return 0;
+        if (!(mixed || device) || !nct || nct == 1 || WT == 1) return 0;
         const int ngroups = (nct + WT - 1) / WT;
-        return ngroups >= U ? (int)(round_up(ngroups) / U) : 0;
+        return device || ngroups >= U ? (int)(round_up(ngroups) / U) : 0;
     };
     auto quad_visible = [&](int s, int qd) -> int {
         const int rows = cu_seqlens[s + 1] - cu_seqlens[s];
@@ -2168,11 +2300,26 @@ extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const 
         return std::max(1, std::min((kv_lens[s] + 15) / 16, last_pos / 16 + 1));
     };
     double quad_w = 1.0;
-    if (mixed) {
+    const int max_range = device ? INT_MAX : mf::kMaxItemTiles;
+    if (mixed || device) {
         int64_t visible = 0;
         for (int s = 0; s < num_seqs; ++s)
             for (int qd = 0, nq = quads(s); qd < nq; ++qd) visible += (int64_t)Hkv * quad_visible(s, qd);
         quad_w = std::max((double)std::max(PW, 1), (double)visible / (2.0 * kPlanCUs));
+        if (device && !mixed) {
+            // About two workgroups per compute unit, of at least 16 tiles;
+            // where that makes ranges longer than 96 tiles, about four, of at
+            // least 96. Measured, us at 8 / 16 / 24 / 32 / 48 / 64 / 128 tiles
+            // per range and uncut: one chunk of 256 rows after 6144 keys, 15/5
+            // heads x 64 33.6 / 27.3 / 24.3 / 24.0 / 24.7 / 29.2 / 38 / 88 (rule
+            // 23), 40/8 x 128 99 / 71 / 62 / 66 / 51 / 58 / 79 / 202 (64); 1024
+            // fresh rows, x 64 19.8 / 18.1 / 19.1 / 21.4 / 21.0 uncut (16), x 128
+            // 50 / 36 / 36 / 41 / 45 uncut (20); 2 chunks of about 850 rows
+            // after 4000 keys x 128 714 / 449 / 374 / 335 / 301 / 291 / 295 / 292
+            // (200: 284).
+            quad_w = std::max(16.0, (double)visible / (2.0 * kPlanCUs));
+            if (quad_w > 96) quad_w = std::max(96.0, (double)visible / (4.0 * kPlanCUs));
+        }
     }
     // Partition counts per (sequence, quad), then at most two wide
     // workgroups per CU: rounding can leave a few more, and with every CU
@@ -2181,7 +2328,7 @@ extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const 
     // grow the least. C2: 530 -> 510 workgroups, engine layer 42.1-42.3 us
     // against 42.7-42.9.
     std::vector<std::vector<int>> qparts(num_seqs);
-    if (mixed) {
+    if (mixed || device) {
         int64_t total = 0;
         for (int s = 0; s < num_seqs; ++s) {
             const int nq = quads(s);
@@ -2189,17 +2336,17 @@ extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const 
             for (int qd = 0; qd < nq; ++qd) {
                 const int v = quad_visible(s, qd);
                 const int n = std::max(1, (int)std::lround(v / quad_w));
-                qparts[s][qd] = std::max(n, (v + mf::kMaxItemTiles - 1) / mf::kMaxItemTiles);
+                qparts[s][qd] = std::max<int>(n, ((int64_t)v + max_range - 1) / max_range);
                 total += (int64_t)Hkv * qparts[s][qd];
             }
         }
-        while (total > 2 * kPlanCUs) {
+        while (mixed && total > 2 * kPlanCUs) {
             int bs = -1, bq = -1;
             double best = 1e300;
             for (int s = 0; s < num_seqs; ++s)
                 for (int qd = 0; qd < (int)qparts[s].size(); ++qd) {
                     const int n = qparts[s][qd], v = quad_visible(s, qd);
-                    if (n <= 1 || (v + n - 2) / (n - 1) > mf::kMaxItemTiles) continue;
+                    if (n <= 1 || (v + n - 2) / (n - 1) > max_range) continue;
                     const double grown = (double)v / (n - 1);
                     if (grown < best) {
                         best = grown;
@@ -2307,7 +2454,13 @@ extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const 
                         }
                     }
                     for (int p = 0; p < n; ++p) {
-                        const int k0 = (int)((int64_t)p * v / n), k1 = (int)((int64_t)(p + 1) * v / n);
+                        const int k0 = (int)((int64_t)p * v / n);
+                        // v counts the keys of distinct positions that end the
+                        // context; rows that share a position (the operator's
+                        // non-causal queries) see more, so a device plan's last
+                        // range runs to the context's end and the kernel stops
+                        // where its rows do
+                        const int k1 = device && p + 1 == n ? tiles : (int)((int64_t)(p + 1) * v / n);
                         for (int k = 0; k < U; ++k) {
                             const int gi = qd * U + k;
                             Item o{};
@@ -2486,7 +2639,7 @@ extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const 
             const Item& b = wunits[y][0];
             // one key range; in a mixed plan one (sequence, kv head), whose
             // quads' ranges overlap
-            return a[0] == b[0] && a[1] == b[1] && (mixed || (a[4] == b[4] && a[5] == b[5]));
+            return a[0] == b[0] && a[1] == b[1] && (mixed || device || (a[4] == b[4] && a[5] == b[5]));
         };
         // run r holds units [run_begin[r], run_begin[r + 1])
         std::vector<size_t> run_begin;
@@ -2544,6 +2697,24 @@ extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const 
         emit(wunits, n_narrow);
     }
     return MF_OK;
+}
+}  // namespace
+
+extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
+                                 int num_q_heads, int num_kv_heads, int head_dim, int dtype,
+                                 int partition_tiles, int32_t* items, int64_t items_capacity,
+                                 int32_t* merges, int64_t merges_capacity, int64_t* counts) {
+    return attention_plan(num_seqs, cu_seqlens, kv_lens, num_q_heads, num_kv_heads, head_dim, dtype,
+                          partition_tiles, 0, items, items_capacity, merges, merges_capacity, counts);
+}
+
+extern "C" int mf_attention_plan_device(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
+                                        int num_q_heads, int num_kv_heads, int head_dim, int dtype, int num_cus,
+                                        int32_t* items, int64_t items_capacity, int32_t* merges,
+                                        int64_t merges_capacity, int64_t* counts) {
+    if (num_cus <= 0) return MF_ERR_ARG;
+    return attention_plan(num_seqs, cu_seqlens, kv_lens, num_q_heads, num_kv_heads, head_dim, dtype, 0, num_cus,
+                          items, items_capacity, merges, merges_capacity, counts);
 }
 
 // Slice plan for a large decode launch (attn_slice_kernel). The sequences'

@@ -73,7 +73,8 @@ def packed_forward(model, pool, tokens: Sequence[Sequence[int]], starts: Sequenc
     flat_tokens = np.fromiter((tok for run in tokens for tok in run), dtype=np.int32)
     nat.check_pack_entries(ent, flat_tables, len(flat_tokens), T, pool.num_blocks)
     items, merges, counts = nat.plan_attention_host(cu.tolist(), kv_lens, model.config.num_attention_heads,
-                                                    spec.num_kv_heads, spec.head_dim, pool.key_pool.dtype)
+                                                    spec.num_kv_heads, spec.head_dim, pool.key_pool.dtype,
+                                                    num_cus=nat.device_cus(spec.device))
     keep_np = np.asarray(list(keep_rows), dtype=np.int64)
     # descriptors, tables, tokens, the attention plan and the kept rows cross
     # to the device in one copy

@@ -1,0 +1,82 @@
+"""mf_attention_plan_device: every tile of every column is planned exactly once
+-- up to the context's end, since rows that share a position see past the
+causal estimate -- and every partial slot is merged exactly once, over the
+shapes the general planner takes; where it has no rule of its own (fp32, padded
+head_dim) it is that planner."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from memforge_amd import _native as nat
+
+
+def _cover(items, merges, counts, q_lens, kv, hq, hkv, d):
+    G = hq // hkv
+    n_narrow, n_wide = int(counts[0]), int(counts[1])
+    assert n_narrow % 4 == 0 and n_wide % 4 == 0 and items.shape[0] == n_narrow + n_wide
+    cu = np.concatenate([[0], np.cumsum(q_lens)])
+    cover, slots = {}, {}
+    for i, it in enumerate(items):
+        s, h, c0, nct, kt0, kt1, slot, _, row0, rows, kvl, coop = (int(x) for x in it)
+        if nct == 0:
+            assert slot == -1
+            continue
+        assert (row0, rows, kvl) == (int(cu[s]), q_lens[s], kv[s])
+        for c in range(c0, c0 + nct):
+            cover.setdefault((s, h, c), []).append((kt0, kt1))
+            if slot >= 0 and not (coop and i % 4):
+                assert slot + c - c0 not in slots
+                slots[slot + c - c0] = (s, h, c)
+    for s, (q, n) in enumerate(zip(q_lens, kv)):
+        for h in range(hkv):
+            for c in range((q * G + 15) // 16 if n else 0):
+                ranges = sorted(r for r in cover.pop((s, h, c)) if r[1] > r[0])
+                assert ranges[0][0] == 0 and ranges[-1][1] == (n + 15) // 16
+                assert all(a[1] == b[0] for a, b in zip(ranges, ranges[1:]))
+    assert not cover
+    named = {}
+    for m in merges:
+        s, h, c, n, slot0, stride = (int(x) for x in m[:6])
+        for p in range(n):
+            assert slots[slot0 + p * stride] == (s, h, c) and slot0 + p * stride not in named
+            named[slot0 + p * stride] = True
+    assert len(named) == len(slots)
+    assert int(counts[3]) >= len(slots) * 16 * (max(d, 32) + 2)
+
+
+@pytest.mark.parametrize("hq,hkv,d,dtype", [(15, 5, 64, torch.bfloat16), (40, 8, 128, torch.float16),
+                                            (16, 4, 32, torch.bfloat16), (8, 2, 256, torch.bfloat16),
+                                            (15, 5, 64, torch.float32), (8, 8, 16, torch.bfloat16)])
+@pytest.mark.parametrize("cus", [1, 8, 256])
+def test_device_plans_cover_every_tile_once(hq, hkv, d, dtype, cus):
+    rng = np.random.default_rng(cus + d)
+    shapes = [([1] * 9, [int(x) for x in rng.integers(1, 9000, 9)]), ([5] * 7, [int(x) for x in rng.integers(5, 3000, 7)]),
+              ([1, 40, 7, 0, 130, 1, 3], [700, 2100, 7, 0, 5000, 1, 33]), ([512], [6656]), ([33], [33]),
+              ([20, 300, 1024], [20, 2348, 1024])]
+    for q_lens, kv in shapes:
+        cu = np.concatenate([[0], np.cumsum(q_lens)]).tolist()
+        made = nat.plan_attention_host(cu, kv, hq, hkv, d, dtype, num_cus=cus)
+        _cover(*made, q_lens, kv, hq, hkv, d)
+        if dtype == torch.float32 or d == 16:
+            same = nat.plan_attention_host(cu, kv, hq, hkv, d, dtype)
+            assert all(np.array_equal(a, b) for a, b in zip(made, same))
+
+
+def test_device_plans_keep_wide_workgroups_shared_and_leave_full_grids_uncut():
+    cu, kv = [0, 2048, 4096], [8000, 5000]
+    items, merges, counts = nat.plan_attention_host(cu, kv, 40, 8, 128, torch.bfloat16, num_cus=256)
+    assert merges.shape[0] == 0 and int((items[:, 5] - items[:, 4]).max()) == 500
+    items, merges, counts = nat.plan_attention_host([0, 20, 31], [900, 3000], 15, 5, 64, torch.bfloat16, num_cus=256)
+    assert int(counts[0]) == 0 and merges.shape[0] > 0  # few workgroups: ranges are cut
+    for u in range(0, items.shape[0], 4):
+        assert len({tuple(x[[0, 1, 4, 5]]) for x in items[u:u + 4]}) == 1
+
+
+def test_device_plan_refuses_a_device_without_compute_units():
+    a = np.array([0, 1], dtype=np.int32)
+    counts = np.zeros(4, dtype=np.int64)
+    assert nat.lib().mf_attention_plan_device(1, a.ctypes.data, a[1:].ctypes.data, 2, 1, 64, 2, 0, None, 0, None, 0,
+                                              counts.ctypes.data) == -1
