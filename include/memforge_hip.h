@@ -355,7 +355,8 @@ int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv
  * planner: the same records, run by the same entry points, with the same
  * results up to fp32 summation order. Wide workgroups (16-bit types, head_dim
  * a kernel size) are cut by column quads, for about two or four workgroups per
- * compute unit, with ranges of any length. No counterpart
+ * compute unit, with ranges of any length; decode rows that leave compute
+ * units idle run as more and shorter cooperative units. No counterpart
  * in the reference: it serves the launch, not the data path. */
 int mf_attention_plan_device(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
                              int num_q_heads, int num_kv_heads, int head_dim, int dtype, int num_cus,

@@ -2236,6 +2236,54 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
     // each K/V tile through LDS. Shorter runs are pooled and packed kWaves to
     // a workgroup, each wave on its own keys.
     const int U = mf::kWaves;
+    // Decode steps planned for a device (one row a sequence, one column tile
+    // each) that the general partition leaves with fewer than two workgroups
+    // per compute unit. There the longest chain of tiles sets the time, so
+    // ranges run as cooperative units from a few tiles on: above 4 / 16 / 32
+    // tiles with up to one / two / more (sequence, kv head) pairs per compute
+    // unit. At 256-byte rows a range is cut where the longest holds more than 80
+    // tiles -- below, the merge launch costs more than its chain -- into units of
+    // about total / (1.8 x compute units) tiles, at least 32 and at most 72: two
+    // workgroups of a unit per compute unit and one round of them. At 128-byte
+    // rows, whose tiles chain three times as fast, a step with ranges of more
+    // than 100 tiles keeps the general plan, which cuts those well (59 sequences
+    // of up to 2800 keys at 9/3 x 64 19.6 us against 22.7 cut as above).
+    // Measured, us, general plan then this one: 64 sequences of up to 1152 keys
+    // at 15/5 x 64 17.4, 15.3 (units of 64 tiles and merges 19.2); at 40/8 x 128
+    // 4 of 8192 to 24576 84, 66 (units of 128 tiles 76, 256 84); 16 of 500 to
+    // 4000 73, 45 (uncut 71); 64 of 200 to 3000 119, 70 (uncut 85). A lone
+    // wave's tile takes 0.33 us at 4 KB of K and V, 0.95 at 8 KB.
+    int single_max = P;
+    double unit_tiles = 0;  // tiles per unit of a cut range (0: the general partition)
+    if (num_cus > 0 && partition_tiles <= 0 && !mixed) {
+        int64_t pairs = 0, tiles_all = 0, singles = 0, units = 0;
+        int longest = 0;
+        bool decode = true;
+        for (int s = 0; s < num_seqs; ++s) {
+            const int nct = col_tiles(s);
+            if (!nct) continue;
+            decode = decode && nct == 1 && cu_seqlens[s + 1] - cu_seqlens[s] == 1;
+            const int T = (kv_lens[s] + 15) / 16;
+            pairs += Hkv;
+            tiles_all += (int64_t)Hkv * T;
+            longest = std::max(longest, T);
+            if (T > P) units += (int64_t)Hkv * ((T + U * P - 1) / (U * P));
+            else singles += Hkv;
+        }
+        if (decode && units + singles / U < 2 * (int64_t)num_cus) {
+            const bool long_rows = DP * mf::dtype_size(dtype) >= 256;
+            if (long_rows || longest <= 100) {
+                single_max = pairs <= num_cus ? 4 : pairs <= 2 * (int64_t)num_cus ? 16 : 32;
+                unit_tiles = long_rows && longest > 80
+                                 ? std::min(72.0, std::max(32.0, (double)tiles_all / (1.8 * num_cus)))
+                                 : 1e9;
+            }
+        }
+    }
+    auto decode_units = [&](int tiles) {
+        const int n = std::max(1, (int)std::lround(tiles / unit_tiles));
+        return std::max(n, (tiles + U * mf::kMaxItemTiles - 1) / (U * mf::kMaxItemTiles));
+    };
     auto round_up = [&](int64_t n) { return (n + U - 1) / U * U; };
     // key partitions of sequence s: count, and the start of partition p
     // (narrow cooperative ranges are balanced; the rest are Q-tile strides).
@@ -2245,8 +2293,9 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
     // partition).
     auto partitions = [&](int s, bool narrow, int& Q, bool& coop) {
         const int tiles = (kv_lens[s] + 15) / 16;
-        coop = narrow && tiles > P;
+        coop = narrow && tiles > single_max;
         Q = narrow ? (coop ? U * P : P) : PW;
+        if (narrow && unit_tiles > 0) return coop ? decode_units(tiles) : 1;
         if (!narrow && tiles > PW) {
             const int np = (tiles + PW - 1) / PW;
             Q = (tiles + np - 1) / np;
@@ -2307,8 +2356,9 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
             for (int qd = 0, nq = quads(s); qd < nq; ++qd) visible += (int64_t)Hkv * quad_visible(s, qd);
         quad_w = std::max((double)std::max(PW, 1), (double)visible / (2.0 * kPlanCUs));
         if (device && !mixed) {
-            // About two workgroups per compute unit, of at least 16 tiles;
-            // where that makes ranges longer than 96 tiles, about four, of at
+            // About two workgroups per compute unit, of at least 16 tiles (12 at
+            // head_dim 128: 7-row verifies of up to 600 keys at 40/8 18.5 us
+            // against 21.8 at 16); where that makes ranges longer than 96 tiles, about four, of at
             // least 96. Measured, us at 8 / 16 / 24 / 32 / 48 / 64 / 128 tiles
             // per range and uncut: one chunk of 256 rows after 6144 keys, 15/5
             // heads x 64 33.6 / 27.3 / 24.3 / 24.0 / 24.7 / 29.2 / 38 / 88 (rule
@@ -2317,7 +2367,7 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
             // 50 / 36 / 36 / 41 / 45 uncut (20); 2 chunks of about 850 rows
             // after 4000 keys x 128 714 / 449 / 374 / 335 / 301 / 291 / 295 / 292
             // (200: 284).
-            quad_w = std::max(16.0, (double)visible / (2.0 * kPlanCUs));
+            quad_w = std::max(DP >= 128 ? 12.0 : 16.0, (double)visible / (2.0 * kPlanCUs));
             if (quad_w > 96) quad_w = std::max(96.0, (double)visible / (4.0 * kPlanCUs));
         }
     }
@@ -2512,7 +2562,13 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
         for (int p = 0; p < nparts; ++p) {
             const int k0 = part_begin(tiles, nparts, Q, coop, p);
             const int k1 = part_begin(tiles, nparts, Q, coop, p + 1);
-            for (int h = 0; h < Hkv; ++h) {
+            for (int hi = 0; hi < Hkv; ++hi) {
+                // A device's decode units start one kv head on from the last
+                // range's: with 8 heads workgroup b's head would otherwise be b
+                // mod 8, its XCD's number, and an XCD that reads one head of
+                // every row uses one channel in eight of its L2 (67 against 75
+                // us, the 4 long sequences at 64-tile units).
+                const int h = narrow && unit_tiles > 0 ? (hi + p + s) % Hkv : hi;
                 if (narrow) {
                     for (int gi = 0; gi < ngroups; ++gi) {
                         if (!coop) {
