@@ -1031,6 +1031,20 @@ class VerifyResult:
     is_draft: torch.Tensor      # uint8 [B, K+1]
     count: torch.Tensor         # int32 [B]
     num_accepted: torch.Tensor  # int32 [B]
+    packed: Optional[torch.Tensor] = None  # the int32 buffer the four are views of, in the order of ``split``
+
+    @staticmethod
+    def split(packed: torch.Tensor, B: int, K: int) -> "VerifyResult":
+        """The four results as views of a packed buffer (the device one, or its
+        host copy: one transfer for all of them)."""
+        n = B * (K + 1)
+        return VerifyResult(
+            tokens=packed[:n].view(B, K + 1),
+            is_draft=packed[n + 2 * B:].view(torch.uint8)[:n].view(B, K + 1),
+            count=packed[n:n + B],
+            num_accepted=packed[n + B:n + 2 * B],
+            packed=packed,
+        )
 
 
 _VERIFY_WS_BYTES = {}  # (rows, candidates) -> mf_spec_verify_workspace_size
@@ -1076,9 +1090,4 @@ def spec_verify(draft_tokens: torch.Tensor, draft_probs: torch.Tensor, target_lo
         exp_noise.data_ptr(), exp_noise.stride(0), base, base + 4 * (n + 2 * B), base + 4 * n,
         base + 4 * (n + B), ws.data_ptr(), ws_bytes, stream,
     ), "mf_spec_verify")
-    return VerifyResult(
-        tokens=out[:n].view(B, K + 1),
-        is_draft=out[n + 2 * B:].view(torch.uint8)[:n].view(B, K + 1),
-        count=out[n:n + B],
-        num_accepted=out[n + B:n + 2 * B],
-    )
+    return VerifyResult.split(out, B, K)

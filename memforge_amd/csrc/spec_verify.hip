@@ -1,11 +1,11 @@
 // Speculative rejection sampling with caller-supplied randomness.
 //
 // Launch 1 (skipped when the target rows already are probabilities): softmax
-// statistics of logits[b][i][:V] / T. Each row is split into 8192-element
-// chunks, one 256-thread workgroup per (row, chunk), every element loaded once
+// statistics of logits[b][i][:V] / T. Each row is split into chunks of 8192
+// (or 4096) elements, one 256-thread workgroup per (row, chunk), every element loaded once
 // into registers with 16-byte vector loads; the workgroup writes its chunk's
 // max, sum of exp(x - max) and first argmax of the raw logits.
-// Launch 2 (one workgroup per (row, 2048-element chunk)): combines the chunk
+// Launch 2 (one workgroup per (row, chunk of 2048 or 1024)): combines the chunk
 // statistics of the row's K+1 target positions, runs the sequential accept
 // loop over the K candidates in one lane, in double precision, exactly the
 // reference's arithmetic, and takes one pass over its chunk of the stopping
@@ -42,11 +42,20 @@ namespace mf {
 namespace {
 
 constexpr int kStatThreads = 256;
-constexpr int kStatVec = 8;                             // float4 groups per thread per chunk
-constexpr int kChunk = kStatThreads * 4 * kStatVec;    // elements per statistics workgroup
 constexpr int kPassThreads = 256;
-constexpr int kPassVec = 2;                             // float4 groups per thread per pass chunk
-constexpr int kPassChunk = kPassThreads * 4 * kPassVec;  // elements per draw-pass workgroup
+// Elements per statistics and per draw-pass workgroup, from their float4 groups
+// per thread. Calls of many rows take 8 and 2; where that makes at most
+// kFewChunks statistics workgroups -- two per compute unit, the chip half idle
+// and every workgroup's loads and exponentials in one chain -- half of each.
+// Measured on MI355X, graph replays, 8 / 2 against 4 / 1 (us per call): 16 rows
+// of 4 candidates over 49,152 fp32 logits (480 workgroups) 26.5, 24.4; over
+// 32,000 bf16 (320) 25.0, 20.1; one row (30) 20.6, 17.9; 48 rows of 7 (2,304)
+// 42.1, 45.4; 64 rows of 3 over 152,064 (4,864) 99, 145.
+constexpr int kFewChunks = 512;
+constexpr int stat_vec(bool few) { return few ? 4 : 8; }
+constexpr int pass_vec(bool few) { return few ? 1 : 2; }
+constexpr int stat_chunk(bool few) { return kStatThreads * 4 * stat_vec(few); }
+constexpr int pass_chunk(bool few) { return kPassThreads * 4 * pass_vec(few); }
 constexpr int kMaxPositions = 64;                       // K + 1 target positions per row
 constexpr int kStatBatch = 8;                           // chunk statistics loaded per round trip
 
@@ -200,8 +209,9 @@ __device__ void block_argmax(float& v, int& i, float* shv, int* shi) {
     for (int k = 1; k < NW; ++k) argmax_merge(v, i, shv[k], shi[k]);
 }
 
-template <int DT>
+template <int DT, bool FEW>
 __global__ __launch_bounds__(kStatThreads) void row_stats_kernel(VerifyArgs a) {
+    constexpr int kStatVec = stat_vec(FEW), kChunk = stat_chunk(FEW);
     __shared__ float shv[4], shs[4];
     __shared__ int shi[4];
     const int c = blockIdx.x;    // chunk of the row
@@ -388,8 +398,9 @@ __device__ __forceinline__ void accept_row(const VerifyArgs& a, int b, float* s_
 // The draw's pass over one (chunk, row): first-index argmaxes of the three
 // candidate families at the stopping position (residual only when the round
 // rejected), and the chunk's "has mass" bits.
-template <int DT>
+template <int DT, bool FEW>
 __global__ __launch_bounds__(kPassThreads) void draw_kernel(VerifyArgs a) {
+    constexpr int kPassVec = pass_vec(FEW), kPassChunk = pass_chunk(FEW);
     __shared__ float s_max[kMaxPositions], s_sum[kMaxPositions];
     __shared__ int s_arg[kMaxPositions];
     __shared__ int s_stop, s_reject;
@@ -540,8 +551,8 @@ __global__ __launch_bounds__(64) void finish_kernel(VerifyArgs a) {
     a.out_num_accepted[b] = i;
 }
 
-inline int chunks_for(int vocab) { return (vocab + kChunk - 1) / kChunk; }
-inline int pass_chunks_for(int vocab) { return (vocab + kPassChunk - 1) / kPassChunk; }
+inline int chunks_for(int vocab, bool few) { return (vocab + stat_chunk(few) - 1) / stat_chunk(few); }
+inline int pass_chunks_for(int vocab, bool few) { return (vocab + pass_chunk(few) - 1) / pass_chunk(few); }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -557,9 +568,9 @@ inline Layout layout_for(int64_t num_rows, int num_draft) {
     // sized for a vocabulary of up to 2^20 entries
     const int64_t rows = num_rows * (num_draft + 1);
     Layout l;
-    l.st = rows * mf::chunks_for(1 << 20);
+    l.st = rows * mf::chunks_for(1 << 20, true);
     l.rows = num_rows;
-    l.pass = num_rows * mf::pass_chunks_for(1 << 20);
+    l.pass = num_rows * mf::pass_chunks_for(1 << 20, true);
     l.total_bytes = (3 * l.st + 2 * l.rows + 7 * l.pass) * 4 + 256;
     return l;
 }
@@ -589,7 +600,8 @@ extern "C" int mf_spec_verify(int num_rows, int num_draft, int vocab, const int3
     if (!workspace || workspace_bytes < mf_spec_verify_workspace_size(num_rows, num_draft))
         return MF_ERR_WORKSPACE;
     const int64_t nrow = (int64_t)num_rows * (num_draft + 1);
-    const int nchunk = chunks_for(vocab);
+    const bool few = nrow * chunks_for(vocab, false) <= kFewChunks;
+    const int nchunk = chunks_for(vocab, few);
     // a vector load covers 4 elements: 16 bytes of fp32, 8 bytes of bf16/f16
     const int es = target_dtype == MF_F32 ? 4 : 2;
     const bool vec_logits = ((uintptr_t)target_logits % (4 * es)) == 0 && (tl_stride_row % 4) == 0 &&
@@ -598,7 +610,7 @@ extern "C" int mf_spec_verify(int num_rows, int num_draft, int vocab, const int3
                        (aligned16(draft_probs) && (dp_stride_row % 4) == 0 && (dp_stride_pos % 4) == 0);
     const bool vec_e = aligned16(exp_noise) && (noise_stride_row % 4) == 0;
     const Layout l = layout_for(num_rows, num_draft);
-    const int npass = pass_chunks_for(vocab);
+    const int npass = pass_chunks_for(vocab, few);
     float* ws = (float*)workspace;
     float* p = ws;
     auto take = [&](int64_t n) { float* r = p; p += n; return r; };
@@ -627,20 +639,22 @@ extern "C" int mf_spec_verify(int num_rows, int num_draft, int vocab, const int3
                  row_reject, npass, part_best, part_best_i, part_any,
                  vec_logits ? 1 : 0, vec_q ? 1 : 0, vec_e ? 1 : 0};
     hipStream_t st = (hipStream_t)stream;
-    auto run = [&](auto dt_tag) -> int {
+    auto run = [&](auto dt_tag, auto few_tag) -> int {
         constexpr int DT = decltype(dt_tag)::value;
+        constexpr bool FEW = decltype(few_tag)::value;
         if (!target_is_probs) {
-            hipLaunchKernelGGL(row_stats_kernel<DT>, dim3((unsigned)nchunk, (unsigned)nrow), dim3(kStatThreads), 0,
+            hipLaunchKernelGGL((row_stats_kernel<DT, FEW>), dim3((unsigned)nchunk, (unsigned)nrow), dim3(kStatThreads), 0,
                                st, a);
             if (int e = check_launch()) return e;
         }
         const dim3 grid((unsigned)npass, (unsigned)num_rows);
-        hipLaunchKernelGGL((draw_kernel<DT>), grid, dim3(kPassThreads), 0, st, a);
+        hipLaunchKernelGGL((draw_kernel<DT, FEW>), grid, dim3(kPassThreads), 0, st, a);
         if (int e = check_launch()) return e;
         hipLaunchKernelGGL(finish_kernel, dim3((unsigned)num_rows), dim3(64), 0, st, a);
         return check_launch();
     };
-    if (target_dtype == MF_F32) return run(std::integral_constant<int, MF_F32>{});
-    if (target_dtype == MF_BF16) return run(std::integral_constant<int, MF_BF16>{});
-    return run(std::integral_constant<int, MF_F16>{});
+    auto pick = [&](auto dt_tag) { return few ? run(dt_tag, std::true_type{}) : run(dt_tag, std::false_type{}); };
+    if (target_dtype == MF_F32) return pick(std::integral_constant<int, MF_F32>{});
+    if (target_dtype == MF_BF16) return pick(std::integral_constant<int, MF_BF16>{});
+    return pick(std::integral_constant<int, MF_F16>{});
 }

@@ -422,12 +422,15 @@ def resolve_rounds_batched(seq_ids: Sequence[int], candidates: torch.Tensor, dra
     uniforms and exp_noise (B, V) Exp(1) draws, all on the GPU. Row b uses
     u_accept[b][i] for candidate i and exp_noise[b] for its final draw.
     """
-    res = nat.spec_verify(candidates, draft_probs, target_logits, temperature, u_accept, exp_noise)
-    tokens = res.tokens.cpu().tolist()
-    flags = res.is_draft.cpu().tolist()
-    counts = res.count.cpu().tolist()
-    nacc = res.num_accepted.cpu().tolist()
-    cand = candidates.cpu().tolist()
+    # the candidates' copy is queued ahead of the kernels and the four results
+    # come back as the one buffer they share, so the host waits once
+    cand_host = torch.empty(candidates.shape, dtype=candidates.dtype, pin_memory=True)
+    cand_host.copy_(candidates, non_blocking=True)
+    packed = nat.spec_verify(candidates, draft_probs, target_logits, temperature, u_accept, exp_noise).packed.cpu()
+    res = nat.VerifyResult.split(packed, *candidates.shape)
+    tokens, flags = res.tokens.tolist(), res.is_draft.tolist()
+    counts, nacc = res.count.tolist(), res.num_accepted.tolist()
+    cand = cand_host.tolist()
     return [SpeculativeRound(seq_id=int(s), candidates=cand[b], accepted=tokens[b][: counts[b]],
                              is_draft=[bool(x) for x in flags[b][: counts[b]]], num_accepted_draft=nacc[b])
             for b, s in enumerate(seq_ids)]

@@ -206,3 +206,20 @@ def test_vocabularies_past_one_batch_of_chunk_statistics(device, V):
     for agree, seed in ((0.0, 31), (1.0, 32)):
         draft, target, tokens, u, noise = _inputs(seed, 3, 3, V, agree=agree)
         _run_both(device, draft, target, tokens, u, noise, 1.0)
+
+
+@pytest.mark.parametrize("B,V", [(64, 16384), (65, 16384), (64, 8193), (2, 4097), (2, 1023)])
+def test_rounds_of_few_and_many_workgroups(device, B, V):
+    """Both sides of the chunk-size rule (512 statistics workgroups: 64 rows of
+    4 positions over two chunks of 8,192) and the remainders of the smaller
+    chunks, all three read-outs of one transfer included."""
+    draft, target, tokens, u, noise = _inputs(B + V, B, 3, V, agree=0.6)
+    count, nacc = _run_both(device, draft, target, tokens, u, noise, 1.0)
+    from memforge_amd.runtime.batched_speculative import resolve_rounds_batched
+
+    rounds = resolve_rounds_batched(range(B), tokens.to(device), torch.softmax(draft, -1).to(device),
+                                    target.to(device), 1.0, u.to(device), noise.to(device))
+    assert [len(r.accepted) for r in rounds] == count.tolist()
+    assert [r.num_accepted_draft for r in rounds] == nacc.tolist()
+    assert [r.candidates for r in rounds] == tokens.tolist()
+    assert all(r.is_draft == [True] * r.num_accepted_draft + [False] for r in rounds)
