@@ -16,22 +16,33 @@ from memforge_amd import _native as nat
 
 def as_table_list(table) -> List[int]:
     if isinstance(table, torch.Tensor):
-        return [int(x) for x in table.reshape(-1).tolist()]
-    return [int(x) for x in table]
+        table = table.reshape(-1).tolist()
+    return list(map(int, table))
+
+
+def _padded_int64(tables: Sequence[Sequence[int]]) -> np.ndarray:
+    width = max(1, max((len(t) for t in tables), default=1))
+    out = np.zeros((max(1, len(tables)), width), dtype=np.int64)
+    for row, t in zip(out, tables):
+        if len(t):
+            row[: len(t)] = t
+    return out
 
 
 def padded_tables_host(tables: Sequence[Sequence[int]]) -> np.ndarray:
     """Block tables as one zero-padded int32 (B, max_blocks) array."""
-    width = max(1, max((len(t) for t in tables), default=1))
-    out = np.zeros((max(1, len(tables)), width), dtype=np.int32)
-    for i, t in enumerate(tables):
-        if len(t):
-            out[i, : len(t)] = np.asarray(t, dtype=np.int64).astype(np.int32)
-    return out
+    return _padded_int64(tables).astype(np.int32)
 
 
 def padded_tables(tables: Sequence[Sequence[int]], device) -> torch.Tensor:
     return nat.upload([padded_tables_host(tables)], device)[0]
+
+
+def _check_ids(tables, order, need, nblocks: int) -> None:
+    for s, n in zip(order, need):
+        ids = np.asarray(tables[s][:n], dtype=np.int64)
+        if ids.size and (int(ids.min()) < 0 or int(ids.max()) >= nblocks):
+            raise IndexError(f"block table of sequence {s} names a block outside the pool of {nblocks}")
 
 
 def run_varlen(q_rows: torch.Tensor, out_rows: torch.Tensor, pool: nat.PoolView,
@@ -67,14 +78,18 @@ def run_varlen(q_rows: torch.Tensor, out_rows: torch.Tensor, pool: nat.PoolView,
     identity = row_map == list(range(T))
     # every block id the kernel will read must address the pool
     bs, nblocks = pool.block_size, pool.num_blocks
+    need: List[int] = []
     for i, s in enumerate(order):
         keys = kvl[i] if pool_lens is None else min(kvl[i], pool_lens[s])
-        need = (keys + bs - 1) // bs
-        if need > len(tables[s]):
-            raise IndexError(f"sequence {s} needs {need} blocks but its block table has {len(tables[s])}")
-        ids = np.asarray(tables[s][:need], dtype=np.int64)
-        if ids.size and (int(ids.min()) < 0 or int(ids.max()) >= nblocks):
-            raise IndexError(f"block table of sequence {s} names a block outside the pool of {nblocks}")
+        need.append((keys + bs - 1) // bs)
+        if need[i] > len(tables[s]):
+            _check_ids(tables, order[:i], need, nblocks)  # an earlier sequence's bad id is reported first
+            raise IndexError(f"sequence {s} needs {need[i]} blocks but its block table has {len(tables[s])}")
+    tables64 = _padded_int64([tables[s] for s in order])
+    # (the padding's block 0 and the entries past what is read count only if
+    # the whole array is not in range)
+    if int(tables64.min()) < 0 or int(tables64.max()) >= nblocks:
+        _check_ids(tables, order, need, nblocks)
     nat.require_device(q_rows, out_rows, pool.k)
     # a large decode step on 16-token blocks runs as one round of slices
     sliceable = identity and pool_lens is None and pool.block_size == 16
@@ -83,7 +98,7 @@ def run_varlen(q_rows: torch.Tensor, out_rows: torch.Tensor, pool: nat.PoolView,
     # tables, plan, cu/kv lengths, positions, row map and pool lengths cross
     # to the device in one copy (none when the same bytes crossed before on
     # this stream), and the launch addresses them inside that one buffer
-    tables_host = padded_tables_host([tables[s] for s in order])
+    tables_host = tables64.astype(np.int32)
     parts = [tables_host, *nat.plan_upload_parts(items, merges),
              np.asarray(cu + kvl, dtype=np.int32), np.asarray(list(positions), dtype=np.int64)]
     if not identity:
