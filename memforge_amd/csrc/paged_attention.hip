@@ -2241,7 +2241,11 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
     // per compute unit. There the longest chain of tiles sets the time, so
     // ranges run as cooperative units from a few tiles on: above 4 / 16 / 32
     // tiles with up to one / two / more (sequence, kv head) pairs per compute
-    // unit. At 256-byte rows a range is cut where the longest holds more than 80
+    // unit, and always above P, the most a single wave of the general partition
+    // takes (a longer range left to one wave would also lose its tiles past P;
+    // us as four-wave units, then as single waves: 64 sequences of 256 keys at
+    // 15/5 heads x 64 6.4, 8.5; 40 of 256 at 40/8 x 128 12.8, 17.9; 120 of up to
+    // 256 at 9/3 x 64 5.1, 8.1). At 256-byte rows a range is cut where the longest holds more than 80
     // tiles -- below, the merge launch costs more than its chain -- into units of
     // about total / (1.8 x compute units) tiles, at least 32 and at most 72: two
     // workgroups of a unit per compute unit and one round of them. At 128-byte
@@ -2273,7 +2277,7 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
         if (decode && units + singles / U < 2 * (int64_t)num_cus) {
             const bool long_rows = DP * mf::dtype_size(dtype) >= 256;
             if (long_rows || longest <= 100) {
-                single_max = pairs <= num_cus ? 4 : pairs <= 2 * (int64_t)num_cus ? 16 : 32;
+                single_max = std::min(P, pairs <= num_cus ? 4 : pairs <= 2 * (int64_t)num_cus ? 16 : 32);
                 unit_tiles = long_rows && longest > 80
                                  ? std::min(72.0, std::max(32.0, (double)tiles_all / (1.8 * num_cus)))
                                  : 1e9;

@@ -79,17 +79,42 @@ def test_device_plan_refuses_a_device_without_compute_units():
 
 
 @pytest.mark.parametrize("heads,kv,single,cut", [
-    ((15, 5, 64), [500], 4, False), ((15, 5, 64), [1152] * 64, 16, False),
+    ((15, 5, 64), [500], 4, False), ((15, 5, 64), [1152] * 64, 4, False),
     ((40, 8, 128), [1280] * 8, 4, False), ((40, 8, 128), [16000] * 2, 4, True),
 ])
 def test_device_decode_plans_run_ranges_as_cooperative_units(heads, kv, single, cut):
     cu = list(range(len(kv) + 1))
-    items, merges, _ = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16, num_cus=256)
+    items, merges, counts = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16, num_cus=256)
     assert (merges.shape[0] > 0) == cut and (items[:, 11] == 1).all()
     if not cut:
         assert items.shape[0] == 4 * heads[1] * len(kv)
-    short, _, counts = nat.plan_attention_host(cu, [16 * single] * len(kv), *heads, torch.bfloat16, num_cus=256)
+    _cover(items, merges, counts, [1] * len(kv), kv, *heads)
+    short, none, counts = nat.plan_attention_host(cu, [16 * single] * len(kv), *heads, torch.bfloat16, num_cus=256)
     assert (short[:, 11] == 0).all() and int(counts[2]) == 0
+    _cover(short, none, counts, [1] * len(kv), [16 * single] * len(kv), *heads)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("heads", [(15, 5, 64), (9, 3, 64), (40, 8, 128), (32, 32, 64)])
+def test_device_decode_plans_reach_the_newest_key(heads, dtype):
+    """Batches and contexts on both sides of every limit of the decode rule
+    (pairs per compute unit, tiles of a single wave, rows that are cut): every
+    range is planned to its last tile."""
+    rng = np.random.default_rng(heads[0])
+    for b in (1, 2, 7, 8, 32, 33, 40, 51, 52, 64, 85, 100, 102, 103, 170, 171, 256):
+        for n in (1, 15, 17, 64, 65, 129, 256, 257, 500, 513, 1280, 1600, 2048):
+            mixed = [int(x) for x in rng.integers(1, n + 1, b)]
+            for kv in ([n] * b, mixed):
+                made = nat.plan_attention_host(list(range(b + 1)), kv, *heads, dtype, num_cus=256)
+                items = made[0]
+                ends = np.zeros((b, heads[1]), dtype=np.int64)
+                held = np.zeros((b, heads[1]), dtype=np.int64)
+                live = items[items[:, 3] > 0]
+                np.maximum.at(ends, (live[:, 0], live[:, 1]), live[:, 5])
+                np.add.at(held, (live[:, 0], live[:, 1]), live[:, 5] - live[:, 4])
+                tiles = (np.asarray(kv) + 15) // 16
+                assert (ends == tiles[:, None]).all() and (held == tiles[:, None]).all(), (b, n)
+        _cover(*made, [1] * b, kv, *heads)
 
 
 def test_device_decode_plans_leave_full_grids_and_verify_rows_to_the_general_planner():

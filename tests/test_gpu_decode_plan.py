@@ -1,0 +1,93 @@
+"""Decode steps planned for a device (mf_attention_plan_device) through the
+entry points that use such plans, against the float64 oracle and, for whole
+graphed steps, plain transformers attention."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from memforge_amd import _native as nat
+from memforge_amd.kernels.varlen_attention import paged_attention_varlen
+from oracle import attention as oatt
+from tests.gpu_helpers import pad_tables, random_tables, to_np64
+from tests.tiny_models import tiny_llama
+
+pytestmark = pytest.mark.gpu
+
+# the attention tests' tolerances on N(0,1) values: 2^-8 and 2^-11 relative on
+# P and the output, and fp32 sums
+TOL = {torch.bfloat16: 2e-2, torch.float16: 4e-3, torch.float32: 1e-5}
+
+
+def _decode_case(batch, keys, hq, hkv, d, dtype):
+    gen = torch.Generator().manual_seed(batch + keys)
+    kv = [keys] * batch
+    blocks = batch * ((keys + 15) // 16) + 3
+    tables = random_tables(gen, blocks, kv, 16)
+    kp = torch.randn((blocks, 16, hkv, d), generator=gen).to(dtype)
+    vp = torch.randn((blocks, 16, hkv, d), generator=gen).to(dtype)
+    q = torch.randn((batch, hq, d), generator=gen).to(dtype)
+    want = oatt.varlen_attention(to_np64(q.permute(1, 0, 2)), to_np64(kp), to_np64(vp), tables, list(range(batch)),
+                                 [keys - 1] * batch, 16)
+    return kv, tables, kp, vp, q, want
+
+
+# More (sequence, kv head) pairs than compute units and contexts of more tiles
+# than the general partition gives one wave.
+SHORT = [(64, 256, 15, 5, 64, torch.bfloat16), (100, 250, 9, 3, 64, torch.float32),
+         (40, 256, 40, 8, 128, torch.float16)]
+
+
+@pytest.mark.parametrize("batch,keys,hq,hkv,d,dtype", SHORT)
+def test_batched_decodes_of_short_contexts_attend_every_key(device, batch, keys, hq, hkv, d, dtype):
+    kv, tables, kp, vp, q, want = _decode_case(batch, keys, hq, hkv, d, dtype)
+    dk, dv, dq = kp.to(device), vp.to(device), q.to(device)
+    got = paged_attention_varlen(dq.permute(1, 0, 2).unsqueeze(0), dk.unsqueeze(0), dv.unsqueeze(0), 0, tables,
+                                 list(range(batch)), [keys - 1] * batch, 16)
+    assert np.abs(to_np64(got[0]) - want).max() <= TOL[dtype]
+    # the same step with its newest rows written in flight
+    slots = [t[(keys - 1) // 16] * 16 + (keys - 1) % 16 for t in tables]
+    new_k, new_v = dk.view(-1, hkv, d)[slots].clone(), dv.view(-1, hkv, d)[slots].clone()
+    dk.view(-1, hkv, d)[slots] = float("nan")
+    dv.view(-1, hkv, d)[slots] = float("nan")
+    out = torch.full_like(dq, float("nan"))
+    plan = nat.plan_attention(list(range(batch + 1)), kv, hq, hkv, d, dtype, device)
+    nat.paged_attention_kv_write(
+        dq, out, nat.PoolView.from_bshd(dk, dv), pad_tables(tables, device),
+        torch.arange(batch + 1, dtype=torch.int32, device=device), torch.tensor(kv, dtype=torch.int32, device=device),
+        torch.full((batch,), keys - 1, dtype=torch.int64, device=device), plan, d ** -0.5, hkv, new_k, new_v,
+        torch.tensor(slots, dtype=torch.int64, device=device))
+    assert np.abs(to_np64(out.permute(1, 0, 2)) - want).max() <= TOL[dtype]
+
+
+def test_graphed_decodes_of_short_contexts_attend_every_key(device):
+    """A whole graphed step of 12 sequences of 256 keys, 32 kv heads, against
+    transformers' own attention over the same cached keys."""
+    from transformers.cache_utils import DynamicCache
+
+    from memforge_amd.runtime.graphed_paged_decode import GraphedPagedDecoder
+    from memforge_amd.runtime.kv_pool import ModelKVSpec, PagedKVPool
+
+    batch, ctx, layers = 12, 255, 2
+    model = tiny_llama(num_layers=layers, heads=32, kv_heads=32, head_dim=16)
+    pool = PagedKVPool(ModelKVSpec.from_config(model.config, torch.float32, "cuda:0"), batch * 16 + 4, 16)
+    gen = torch.Generator().manual_seed(3)
+    pool.key_pool.copy_(torch.randn(pool.key_pool.shape, generator=gen).to(device))
+    pool.value_pool.copy_(torch.randn(pool.value_pool.shape, generator=gen).to(device))
+    tables = random_tables(gen, batch * 16 + 4, [ctx + 1] * batch, 16)
+    tokens = [7 + 3 * i for i in range(batch)]
+    cache = DynamicCache()
+    slots = torch.tensor([[t[p // 16] * 16 + p % 16 for p in range(ctx)] for t in tables], device=device)
+    for i in range(layers):
+        k, v = (p[i].reshape(-1, 32, 16)[slots].permute(0, 2, 1, 3).contiguous()
+                for p in (pool.key_pool, pool.value_pool))
+        cache.update(k, v, i)
+    with torch.no_grad():
+        want = model(input_ids=torch.tensor(tokens, device=device).view(batch, 1),
+                     position_ids=torch.full((batch, 1), ctx, device=device), past_key_values=cache,
+                     use_cache=True).logits[:, -1]
+    dec = GraphedPagedDecoder(model, pool, max_batch=16, max_model_len=300)
+    for _ in range(3):  # the same step again: every replay rewrites the same rows
+        torch.testing.assert_close(dec.step(tokens, [ctx] * batch, tables), want, atol=2e-5, rtol=1e-4)
