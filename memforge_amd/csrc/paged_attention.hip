@@ -2585,10 +2585,12 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
                         // candidates, loaded key by key), the last wave counts
                         // MF_TAIL_WAVE_TILES more tiles than it has, so the
                         // others take them and the unit's waves reach its
-                        // LDS combine together.
+                        // LDS combine together -- as far as a wave's
+                        // block-table registers go.
                         const int n = k1 - k0;
                         const int rows = cu_seqlens[s + 1] - cu_seqlens[s];
-                        const int extra = (k1 == tiles && rows > 1) ? MF_TAIL_WAVE_TILES : 0;
+                        const int extra = (k1 == tiles && rows > 1)
+                                              ? std::min(MF_TAIL_WAVE_TILES, U * mf::kMaxItemTiles - n) : 0;
                         auto cut = [&](int w) {
                             return w >= U ? k1 : std::min(k1, k0 + (int)((int64_t)w * (n + extra) / U));
                         };

@@ -124,3 +124,18 @@ def test_device_decode_plans_leave_full_grids_and_verify_rows_to_the_general_pla
         a = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16, num_cus=256)
         b = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16)
         assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("cus,partition", [(0, 128), (0, 0), (256, 0)])
+@pytest.mark.parametrize("hq,hkv,d,rows", [(40, 8, 128, 2), (15, 5, 64, 5)])
+def test_single_column_items_fit_their_block_table_registers(cus, partition, hq, hkv, d, rows):
+    """A wave holds the block-table entries of 128 tiles. The cut that gives a
+    verify unit's last wave fewer tiles must leave the others no more than that,
+    up to units of 512 tiles."""
+    for tiles in (500, 506, 507, 509, 510, 511, 512, 1014, 1017, 1024):
+        kv = [tiles * 16 - 3] * 32
+        cu = [rows * i for i in range(33)]
+        made = nat.plan_attention_host(cu, kv, hq, hkv, d, torch.bfloat16, partition, num_cus=cus)
+        narrow = made[0][:int(made[2][0])]
+        assert narrow.shape[0] and int((narrow[:, 5] - narrow[:, 4]).max()) <= nat.MAX_ITEM_TILES, tiles
+        _cover(*made, [rows] * 32, kv, hq, hkv, d)

@@ -684,3 +684,34 @@ def test_item_counts_are_whole_workgroups(device):
     counted = nat.CountedPlan(5, 3, 1, 1024, device)
     assert (counted.cap_narrow, counted.cap_wide) == (8, 4)
     assert counted.items.shape[0] == 12
+
+
+@pytest.mark.parametrize("tiles", [507, 510, 512])
+def test_longest_verify_unit_reads_every_tile_through_its_own_block(device, tiles):
+    """A cooperative unit of up to 512 tiles whose rows are a verify's: each key
+    in turn -- around the first wave's last tiles and at both ends -- holds all
+    of the attention, so the output is that key's value."""
+    from memforge_amd import _native as nat
+
+    gen = torch.Generator().manual_seed(tiles)
+    hq, hkv, d, rows, bs = 4, 1, 64, 2, 16
+    ctx = tiles * bs - 7
+    kv = ctx + rows
+    tables = random_tables(gen, tiles + 2, [kv], bs)
+    vp = torch.randn((tiles + 2, bs, hkv, d), generator=gen).to(torch.bfloat16).to(device)
+    kp = torch.zeros_like(vp)
+    q = torch.full((rows, hq, d), 4.0, dtype=torch.bfloat16, device=device)
+    nk, nv = torch.zeros((rows, hkv, d), dtype=torch.bfloat16, device=device), vp[0, :rows].clone()
+    cu = [0, rows]
+    plan = nat.plan_attention(cu, [kv], hq, hkv, d, torch.bfloat16, device, 128)
+    args = (nat.PoolView.from_bshd(kp, vp), torch.tensor([tables[0]], dtype=torch.int32, device=device),
+            torch.tensor(cu, dtype=torch.int32, device=device), torch.tensor([kv], dtype=torch.int32, device=device),
+            torch.tensor([ctx, ctx + 1], dtype=torch.int64, device=device), plan, d ** -0.5, hkv)
+    for key in (0, 127 * bs + 3, 128 * bs, 129 * bs - 1, 129 * bs, 130 * bs - 1, 130 * bs, 258 * bs, ctx - 1):
+        kp.zero_()
+        slot = (tables[0][key // bs], key % bs)
+        kp[slot] = 4.0  # score 128 against 0
+        out = torch.full_like(q, float("nan"))
+        nat.paged_attention(q, out, *args, pool_lens=torch.tensor([ctx], dtype=torch.int32, device=device),
+                            new_k_rows=nk, new_v_rows=nv)
+        assert torch.equal(out, vp[slot].expand(rows, hq, d)), key
