@@ -1199,8 +1199,23 @@ __device__ __forceinline__ void ld_lds16_base(const char* base_, uint32_t lane_o
 // 32 KB of LDS a workgroup), 373 us against 403 with two and 64-key stages;
 // two score chains at a time took 430 against 436. Scalar registers count too:
 // a base computed for every load apart, with a branch each, took 630 us.
+//
+// cols holds the first column tile and the tile count of the workgroup's four
+// items, in scalar registers: only the block table's round trip stands before
+// the first stage. Two to three more did -- the other items' columns by vector
+// loads, and a wait for every load in flight behind each test of the row map --
+// which beside decode streams cost a mixed step up to 14%. Graph replays, us,
+// before and after (and with the 16x16 loop): 2 chunks of 512 rows and 24
+// decodes of up to 4700 keys at 15/5 heads x 64 30.6, 26.5 (26.0); 1 chunk of
+// 370 and 29 decodes of up to 1150 15.1, 13.6 (13.5); 4 chunks of 512 and 28
+// decodes of up to 4096 29.4, 28.7 (31.5); 60 decodes of up to 500 keys and 4
+// chunks of about 100 16.0, 15.1 (14.3); 16 prompts of up to 1024 31.5, 30.0
+// (35.8). The wave's own item is read again rather than kept: its registers,
+// held over the caller's comparison, made the 256-byte kernel spill scalars in
+// its loop (two chunks of 2048 rows 409 us against 397).
 template <int DT, int DP, bool TAIL>
-__device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int block) {
+__device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int block,
+                                               const int (&cols)[kWaves][2]) {
     constexpr int RB = DP * 2;       // bytes of one key row
     constexpr int NCH = RB / 16;     // 16-byte chunks per row
     constexpr int KEYS = wide_keys(DP), TS = KEYS / 16;  // keys and 16-key blocks per stage
@@ -1219,8 +1234,7 @@ __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int bloc
     const int lane = threadIdx.x & 63;
     const int hf = lane >> 5;
     const char *k_pool = a.k_pool, *v_pool = a.v_pool, *new_k = a.new_k, *new_v = a.new_v;
-    const int32_t* items = a.items + (int64_t)block * kWaves * MF_PLAN_ITEM_INTS;
-    const int32_t* it = items + wave * MF_PLAN_ITEM_INTS;
+    const int32_t* it = a.items + ((int64_t)block * kWaves + wave) * MF_PLAN_ITEM_INTS;
     const int s = it[0], h = it[1], c0 = it[2], nct = it[3], kt0 = it[4], kt1 = it[5], pslot = it[6], m0 = it[7];
     const int row0 = it[8], nrows = it[9], kv_len = it[10];
     const bool inflight = TAIL || a.pool_lens != nullptr;
@@ -1240,25 +1254,31 @@ __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int bloc
     const int ct = (lane & 31) >> 4, j = lane & 15;
     const int cidx = c0 * 16 + (lane & 31);
     const bool valid = ct < nct && cidx < nrows * a.G;
-    const int crow = valid ? cidx / a.G : 0;
-    const int qhead = h * a.G + (valid ? cidx - crow * a.G : 0);
-    int prow = row0 + crow;
-    if (a.row_map) prow = a.row_map[prow];
-    const int pos = reinterpret_cast<const int32_t*>(a.positions)[2 * (int64_t)prow];
-    const int qpos = valid ? pos : -1;
-    // the positions of the workgroup's other columns (two per lane): how far
-    // its stages run, without an exchange between the waves
-    int wpos = -1;
+    const int col = valid ? cidx : 0;
+    const int crow = (int)((unsigned)col / (unsigned)a.G);
+    const int qhead = h * a.G + col - crow * a.G;
+    // its own row and those of the workgroup's other columns (two per lane),
+    // whose positions say how far the stages run, without an exchange between
+    // the waves. One test of the row map for all three: each one joins behind a
+    // wait for every load in flight.
+    int rows[3] = {row0 + crow, row0, row0};
+    bool other[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        const int32_t* iw = items + (2 * k + hf) * MF_PLAN_ITEM_INTS;
-        const int c = iw[2] * 16 + (lane & 31);
-        const bool v = ct < iw[3] && c < nrows * a.G;
-        int r = row0 + (v ? c / a.G : 0);
-        if (a.row_map) r = a.row_map[r];
-        const int x = reinterpret_cast<const int32_t*>(a.positions)[2 * (int64_t)r];
-        wpos = max(wpos, v ? x : -1);
+        const int c = (hf ? cols[2 * k + 1][0] : cols[2 * k][0]) * 16 + (lane & 31);
+        other[k] = ct < (hf ? cols[2 * k + 1][1] : cols[2 * k][1]) && c < nrows * a.G;
+        rows[1 + k] = row0 + (int)((unsigned)(other[k] ? c : 0) / (unsigned)a.G);
     }
+    if (!TAIL && a.row_map) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) rows[k] = a.row_map[rows[k]];
+    }
+    int rpos[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) rpos[k] = reinterpret_cast<const int32_t*>(a.positions)[2 * (int64_t)rows[k]];
+    const int prow = rows[0];
+    const int qpos = valid ? rpos[0] : -1;
+    const int wpos = max(other[0] ? rpos[1] : -1, other[1] ? rpos[2] : -1);
     uint4 qf[NQ];
 #pragma unroll
     for (int c = 0; c < NQ; ++c) {
@@ -1518,6 +1538,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs& a, const int block) {
         const int num_items = a.dev_count ? *a.dev_count : a.num_items;
         const int32_t* i0 = a.items + (int64_t)block * kWaves * MF_PLAN_ITEM_INTS;
         int32_t key[kWaves][4];
+        int cols[kWaves][2];
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
             const int32_t* iw = i0 + w * MF_PLAN_ITEM_INTS;
@@ -1525,6 +1546,8 @@ __device__ __forceinline__ void attn_block(const AttnArgs& a, const int block) {
             key[w][1] = iw[1];
             key[w][2] = iw[4];
             key[w][3] = iw[5];
+            cols[w][0] = iw[2];
+            cols[w][1] = iw[3];
         }
         bool same = (block + 1) * kWaves <= num_items;
 #pragma unroll
@@ -1532,7 +1555,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs& a, const int block) {
             same = same & (key[w][0] == key[0][0]) & (key[w][1] == key[0][1]) & (key[w][2] == key[0][2]) &
                    (key[w][3] == key[0][3]);
         if (same) {
-            attn_wide_body<DT, DP, TAIL>(a, block);
+            attn_wide_body<DT, DP, TAIL>(a, block, cols);
             return;
         }
     }
