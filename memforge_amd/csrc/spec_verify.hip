@@ -2,7 +2,7 @@
 //
 // Launch 1 (skipped when the target rows already are probabilities): softmax
 // statistics of logits[b][i][:V] / T. Each row is split into chunks of 8192
-// (or 4096) elements, one 256-thread workgroup per (row, chunk), every element loaded once
+// elements, one 256-thread workgroup per (row, chunk), every element loaded once
 // into registers with 16-byte vector loads; the workgroup writes its chunk's
 // max, sum of exp(x - max) and first argmax of the raw logits.
 // Launch 2 (one workgroup per (row, chunk of 2048 or 1024)): combines the chunk
@@ -43,18 +43,21 @@ namespace {
 
 constexpr int kStatThreads = 256;
 constexpr int kPassThreads = 256;
-// Elements per statistics and per draw-pass workgroup, from their float4 groups
-// per thread. Calls of many rows take 8 and 2; where that makes at most
-// kFewChunks statistics workgroups -- two per compute unit, the chip half idle
-// and every workgroup's loads and exponentials in one chain -- half of each.
-// Measured on MI355X, graph replays, 8 / 2 against 4 / 1 (us per call): 16 rows
-// of 4 candidates over 49,152 fp32 logits (480 workgroups) 26.5, 24.4; over
-// 32,000 bf16 (320) 25.0, 20.1; one row (30) 20.6, 17.9; 48 rows of 7 (2,304)
-// 42.1, 45.4; 64 rows of 3 over 152,064 (4,864) 99, 145.
+// Elements per statistics workgroup, the same for every call: a row's softmax
+// sum is added up in this order, so a row's accept test and draw must not depend
+// on how many other rows the call holds.
+constexpr int kStatVec = 8;                          // float4 groups per thread
+constexpr int kChunk = kStatThreads * 4 * kStatVec;
+// Elements per draw-pass workgroup, from its float4 groups per thread (the
+// draw's first-index argmaxes come out the same for any cut). Calls of many rows
+// take 2; where the statistics are at most kFewChunks workgroups -- two per
+// compute unit, the chip half idle -- 1.
+// Measured on MI355X, graph replays, 2 against 1 (us per call): 16 rows
+// of 4 candidates over 49,152 fp32 logits (480 workgroups) 23.9, 23.2; over
+// 32,000 bf16 (320) 23.9, 23.0; one row (30) 21.0, 19.5; 8 of 2 over 1,031 20.7, 18.4; 48 rows of 7
+// (2,304) 42.1 (45.4 with both chunks halved).
 constexpr int kFewChunks = 512;
-constexpr int stat_vec(bool few) { return few ? 4 : 8; }
 constexpr int pass_vec(bool few) { return few ? 1 : 2; }
-constexpr int stat_chunk(bool few) { return kStatThreads * 4 * stat_vec(few); }
 constexpr int pass_chunk(bool few) { return kPassThreads * 4 * pass_vec(few); }
 constexpr int kMaxPositions = 64;                       // K + 1 target positions per row
 constexpr int kStatBatch = 8;                           // chunk statistics loaded per round trip
@@ -209,9 +212,8 @@ __device__ void block_argmax(float& v, int& i, float* shv, int* shi) {
     for (int k = 1; k < NW; ++k) argmax_merge(v, i, shv[k], shi[k]);
 }
 
-template <int DT, bool FEW>
+template <int DT>
 __global__ __launch_bounds__(kStatThreads) void row_stats_kernel(VerifyArgs a) {
-    constexpr int kStatVec = stat_vec(FEW), kChunk = stat_chunk(FEW);
     __shared__ float shv[4], shs[4];
     __shared__ int shi[4];
     const int c = blockIdx.x;    // chunk of the row
@@ -551,7 +553,7 @@ __global__ __launch_bounds__(64) void finish_kernel(VerifyArgs a) {
     a.out_num_accepted[b] = i;
 }
 
-inline int chunks_for(int vocab, bool few) { return (vocab + stat_chunk(few) - 1) / stat_chunk(few); }
+inline int chunks_for(int vocab) { return (vocab + kChunk - 1) / kChunk; }
 inline int pass_chunks_for(int vocab, bool few) { return (vocab + pass_chunk(few) - 1) / pass_chunk(few); }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -568,7 +570,7 @@ inline Layout layout_for(int64_t num_rows, int num_draft) {
     // sized for a vocabulary of up to 2^20 entries
     const int64_t rows = num_rows * (num_draft + 1);
     Layout l;
-    l.st = rows * mf::chunks_for(1 << 20, true);
+    l.st = rows * mf::chunks_for(1 << 20);
     l.rows = num_rows;
     l.pass = num_rows * mf::pass_chunks_for(1 << 20, true);
     l.total_bytes = (3 * l.st + 2 * l.rows + 7 * l.pass) * 4 + 256;
@@ -600,8 +602,8 @@ extern "C" int mf_spec_verify(int num_rows, int num_draft, int vocab, const int3
     if (!workspace || workspace_bytes < mf_spec_verify_workspace_size(num_rows, num_draft))
         return MF_ERR_WORKSPACE;
     const int64_t nrow = (int64_t)num_rows * (num_draft + 1);
-    const bool few = nrow * chunks_for(vocab, false) <= kFewChunks;
-    const int nchunk = chunks_for(vocab, few);
+    const int nchunk = chunks_for(vocab);
+    const bool few = nrow * nchunk <= kFewChunks;
     // a vector load covers 4 elements: 16 bytes of fp32, 8 bytes of bf16/f16
     const int es = target_dtype == MF_F32 ? 4 : 2;
     const bool vec_logits = ((uintptr_t)target_logits % (4 * es)) == 0 && (tl_stride_row % 4) == 0 &&
@@ -643,7 +645,7 @@ extern "C" int mf_spec_verify(int num_rows, int num_draft, int vocab, const int3
         constexpr int DT = decltype(dt_tag)::value;
         constexpr bool FEW = decltype(few_tag)::value;
         if (!target_is_probs) {
-            hipLaunchKernelGGL((row_stats_kernel<DT, FEW>), dim3((unsigned)nchunk, (unsigned)nrow), dim3(kStatThreads), 0,
+            hipLaunchKernelGGL(row_stats_kernel<DT>, dim3((unsigned)nchunk, (unsigned)nrow), dim3(kStatThreads), 0,
                                st, a);
             if (int e = check_launch()) return e;
         }

@@ -223,3 +223,35 @@ def test_rounds_of_few_and_many_workgroups(device, B, V):
     assert [r.num_accepted_draft for r in rounds] == nacc.tolist()
     assert [r.candidates for r in rounds] == tokens.tolist()
     assert all(r.is_draft == [True] * r.num_accepted_draft + [False] for r in rounds)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_row_decides_the_same_alone_and_in_a_large_batch(device, dtype):
+    """A row's accept threshold -- the largest uniform that still accepts its
+    candidate -- is a property of the row, whatever else the call holds. 64
+    rows over 49,152 logits are 768 statistics workgroups, one row 12."""
+    B, V = 64, 49152
+    gen = torch.Generator().manual_seed(5)
+    target = (torch.randn((B, 2, V), generator=gen) * math.sqrt(2.0)).to(dtype).to(device)
+    tokens = torch.randint(0, V, (B, 1), generator=gen, dtype=torch.int32).to(device)
+    # the draft gives its candidate one to two and a half times the target's
+    # probability, so thresholds lie in (0.4, 1)
+    p = torch.softmax(target[:, :1].double(), -1).gather(2, tokens.long().unsqueeze(-1))
+    draft = torch.full((B, 1, V), 1.0 / V, device=device)
+    draft.scatter_(2, tokens.long().unsqueeze(-1), (p * (1.02 + 1.4 * torch.rand(p.shape, generator=gen).to(device))).float())
+    noise = torch.empty((B, V)).exponential_(1.0, generator=gen).to(device)
+
+    def accepted(u, rows=slice(None)):
+        return nat.spec_verify(tokens[rows], draft[rows], target[rows], 1.0, u[rows].contiguous(),
+                               noise[rows]).num_accepted == 1
+
+    lo = torch.full((B, 1), 0.3, device=device).view(torch.int32)
+    hi = torch.full((B, 1), 1.0, device=device).view(torch.int32)
+    assert accepted(lo.view(torch.float32)).all() and not accepted(hi.view(torch.float32)).any()
+    while int((hi - lo).max()) > 1:
+        mid = (lo + hi) // 2
+        ok = accepted(mid.view(torch.float32)).view(B, 1)
+        lo, hi = torch.where(ok, mid, lo), torch.where(ok, hi, mid)
+    moved = [b for b in range(B) if not (bool(accepted(lo.view(torch.float32), slice(b, b + 1)))
+                                         and not bool(accepted(hi.view(torch.float32), slice(b, b + 1))))]
+    assert not moved, f"{len(moved)} of {B} rows decide otherwise alone"
