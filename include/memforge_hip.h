@@ -345,6 +345,11 @@ int mf_paged_attention_noalloc(const void* q, int64_t q_stride_row, int64_t q_st
  * the required sizes). */
 #define MF_PLAN_ITEM_INTS 12
 #define MF_PLAN_MERGE_INTS 8
+/* Set in a merge record's last int (the sequence's rows) and in its items'
+ * merge index (int 7): their partial outputs are fp32 whatever the launch's
+ * type. Device plans only, where decode ranges are cut that mf_attention_plan
+ * would leave to one cooperative unit and its fp32 combine. */
+#define MF_PLAN_FP32_PARTIALS 0x40000000
 int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
                       int num_q_heads, int num_kv_heads, int head_dim, int dtype,
                       int partition_tiles, int32_t* items, int64_t items_capacity,

@@ -307,6 +307,13 @@ __device__ __forceinline__ void store_out_chunk(char* p, const float* vals) {
 // A normalised output is a convex combination of V rows, so it keeps the
 // output type's range; 16-bit partials halve the bytes written and merged
 // against fp32 ones, for one more rounding to that type.
+// Records and items flagged MF_PLAN_FP32_PARTIALS hold the outputs in fp32
+// instead (the slot has the room): a device's decode plan cuts ranges that the
+// general plan runs as one cooperative unit, whose waves combine in fp32, and the
+// cut must not round what the whole unit does not. 16-bit launches of 256-byte
+// rows and more only, as that rule.
+template <int DT, int DP>
+constexpr bool has_fp32_partials() { return DT != MF_F32 && DP >= 128; }
 template <int DT>
 __device__ __forceinline__ char* partial_out(const AttnArgs& a, int64_t slot, int col, int elem) {
     constexpr int ES = DT == MF_F32 ? 4 : 2;
@@ -322,13 +329,13 @@ __device__ __forceinline__ float* partial_ml(const AttnArgs& a, int64_t slot) {
 // Partitions go four at a time with every load of a batch issued before any
 // is used (a batch past the last partition loads only what exists; the
 // condition is wave-uniform), and the running maximum moves batch to batch:
-// a merge of n partitions per wave costs ceil(n/4) memory round trips.
-template <int DT, int DP>
+// a merge of n partitions per wave costs ceil(n/4) memory round trips. PT: the
+// type of the partial outputs; B: partitions per batch.
+template <int DT, int DP, int PT = DT, int B = 4>
 __device__ __forceinline__ void merge_range(const AttnArgs& a, const int32_t* mg, int p0, int pinc, int j,
                                             int dbase, float& mx, float& L, float (&o)[DP / 4]) {
     constexpr int VCH = DP / 16;
-    constexpr int B = 4;
-    constexpr int ES = DT == MF_F32 ? 4 : 2;
+    constexpr int ES = PT == MF_F32 ? 4 : 2;
     constexpr int NW = 4 * VCH * ES / 4;  // words of the lane's chunk
     const int np = mg[3], slot0 = mg[4], sstride = mg[5];
     mx = kMinM;
@@ -342,7 +349,7 @@ __device__ __forceinline__ void merge_range(const AttnArgs& a, const int32_t* mg
         for (int b = 0; b < B; ++b) {
             if (p + b * pinc < np) {
                 const int64_t slot = slot0 + (int64_t)(p + b * pinc) * sstride;
-                ld_words<4 * VCH * ES>(partial_out<DT>(a, slot, j, dbase), raw[b]);
+                ld_words<4 * VCH * ES>(partial_out<PT>(a, slot, j, dbase), raw[b]);
                 const float* ml = partial_ml(a, slot);
                 mb[b] = ml[j];
                 lb[b] = ml[16 + j];
@@ -367,8 +374,8 @@ __device__ __forceinline__ void merge_range(const AttnArgs& a, const int32_t* mg
 #pragma unroll
             for (int e = 0; e < 4 * VCH; ++e) {
                 float v;
-                if constexpr (DT == MF_F32) v = __uint_as_float(raw[b][e]);
-                else v = bits_to_f32<DT>((raw[b][e >> 1] >> (16 * (e & 1))) & 0xffffu);
+                if constexpr (PT == MF_F32) v = __uint_as_float(raw[b][e]);
+                else v = bits_to_f32<PT>((raw[b][e >> 1] >> (16 * (e & 1))) & 0xffffu);
                 o[e] += wl * v;
             }
         }
@@ -378,11 +385,11 @@ __device__ __forceinline__ void merge_range(const AttnArgs& a, const int32_t* mg
 
 // Output row/head of column tile ct's column j, or false for a padding column.
 // mg: a merge record (s, h, column tile, parts, slot0, slot stride, first row,
-// rows)
+// rows and flag)
 __device__ __forceinline__ bool merge_column(const AttnArgs& a, const int32_t* mg, int j, int& prow, int& qhead) {
     const int h = mg[1], ct = mg[2];
     const int row0 = mg[6];
-    const int ncols = mg[7] * a.G;
+    const int ncols = (mg[7] & ~MF_PLAN_FP32_PARTIALS) * a.G;
     const int cidx = ct * 16 + j;
     if (cidx >= ncols) return false;
     const int r = cidx / a.G;
@@ -392,8 +399,9 @@ __device__ __forceinline__ bool merge_column(const AttnArgs& a, const int32_t* m
     return true;
 }
 
-// Single-wave merge of one record (used by the fused in-kernel merge).
-template <int DT, int DP>
+// Single-wave merge of one record. FP32B: partitions per batch of a record of
+// fp32 partials, 0 where the caller's records have none (prefill items).
+template <int DT, int DP, int FP32B = 0>
 __device__ __forceinline__ void merge_tile(const AttnArgs& a, const int32_t* mg, int g, int j) {
     constexpr int VCH = DP / 16;
     constexpr int ES = DT == MF_F32 ? 4 : 2;
@@ -401,7 +409,14 @@ __device__ __forceinline__ void merge_tile(const AttnArgs& a, const int32_t* mg,
     const int dbase = 4 * g * VCH;
     if (!merge_column(a, mg, j, prow, qhead) || dbase >= a.head_dim) return;
     float mx, L, o[4 * VCH];
-    merge_range<DT, DP>(a, mg, 0, 1, j, dbase, mx, L, o);
+    bool merged = false;
+    if constexpr (has_fp32_partials<DT, DP>() && FP32B > 0) {
+        if (mg[7] & MF_PLAN_FP32_PARTIALS) {
+            merge_range<DT, DP, MF_F32, FP32B>(a, mg, 0, 1, j, dbase, mx, L, o);
+            merged = true;
+        }
+    }
+    if (!merged) merge_range<DT, DP>(a, mg, 0, 1, j, dbase, mx, L, o);
     const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
     for (int e = 0; e < 4 * VCH; ++e) o[e] *= inv;
@@ -1068,7 +1083,10 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const int block) {
                     const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
                     for (int c = 0; c < VCH; ++c) o[c] *= inv;
-                    store_elems<DT, VCH>(partial_out<DT>(a, pslot, j, d0), o);
+                    bool fp32 = false;
+                    if constexpr (has_fp32_partials<DT, DP>()) fp32 = (iv1.w & MF_PLAN_FP32_PARTIALS) != 0;
+                    if (fp32) store_elems<MF_F32, VCH>(partial_out<MF_F32>(a, pslot, j, d0), o);
+                    else store_elems<DT, VCH>(partial_out<DT>(a, pslot, j, d0), o);
                     if (g == 0 && wave == 0) {
                         float* ml = partial_ml(a, pslot);
                         ml[j] = M;
@@ -1082,7 +1100,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const int block) {
                 __threadfence();
                 __syncthreads();
                 if (wave == 0) {
-                    const int m0 = iv1.w;
+                    const int m0 = iv1.w & ~MF_PLAN_FP32_PARTIALS;
                     int prev = 0;
                     if (lane == 0) prev = atomicAdd(a.counters + m0, 1);
                     prev = __shfl(prev, 0, 64);
@@ -1090,7 +1108,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const int block) {
                     if (prev == mg0[3] - 1) {
                         __threadfence();
                         if (lane == 0) a.counters[m0] = 0;
-                        merge_tile<DT, DP>(a, mg0, g, j);
+                        merge_tile<DT, DP, 2>(a, mg0, g, j);
                     }
                 }
             }
@@ -1976,7 +1994,7 @@ __global__ __launch_bounds__(64) void merge_kernel(const int32_t* merges, int nu
     load_merge_record(a, merges, mi, num_merges, mg);
     if (mi >= (a.dev_count ? *a.dev_count : num_merges)) return;
     const int lane = threadIdx.x & 63;
-    merge_tile<DT, DP>(a, mg, lane >> 4, lane & 15);
+    merge_tile<DT, DP, (DP > 128 ? 2 : 4)>(a, mg, lane >> 4, lane & 15);
 }
 
 // The split-K merge launch: one single-wave workgroup per record.
@@ -2567,6 +2585,7 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
             continue;
         }
         const int64_t slot0 = slots, merge0 = wm;
+        const int32_t fp32_flag = narrow && unit_tiles > 0 && dtype != MF_F32 ? MF_PLAN_FP32_PARTIALS : 0;
         auto make = [&](int gi, int p, int h, int k0, int k1) {
             const int cg0 = gi * width;
             const int w = std::min(width, nct - cg0);
@@ -2579,7 +2598,7 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
             o[5] = k1;
             o[6] = nparts > 1 ? (int32_t)(slot0 + (int64_t)gi * Hkv * nparts * width + ((int64_t)h * nparts + p) * w)
                               : -1;
-            o[7] = nparts > 1 ? (int32_t)(merge0 + (int64_t)gi * Hkv * width + (int64_t)h * w) : -1;
+            o[7] = nparts > 1 ? (int32_t)(merge0 + (int64_t)gi * Hkv * width + (int64_t)h * w) | fp32_flag : -1;
             o[8] = cu_seqlens[s];
             o[9] = cu_seqlens[s + 1] - cu_seqlens[s];
             o[10] = kv_lens[s];
@@ -2653,7 +2672,7 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
                         o[4] = (int32_t)(group_base + (int64_t)h * nparts * w + o2);
                         o[5] = w;
                         o[6] = cu_seqlens[s];
-                        o[7] = cu_seqlens[s + 1] - cu_seqlens[s];
+                        o[7] = (cu_seqlens[s + 1] - cu_seqlens[s]) | fp32_flag;
                         ++wm;
                     }
                 }

@@ -91,3 +91,39 @@ def test_graphed_decodes_of_short_contexts_attend_every_key(device):
     dec = GraphedPagedDecoder(model, pool, max_batch=16, max_model_len=300)
     for _ in range(3):  # the same step again: every replay rewrites the same rows
         torch.testing.assert_close(dec.step(tokens, [ctx] * batch, tables), want, atol=2e-5, rtol=1e-4)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch,lo,hi,hq,hkv,d", [(8, 1500, 1501, 40, 8, 128), (16, 500, 4000, 40, 8, 128),
+                                                  (3, 9000, 12000, 8, 2, 256)])
+def test_cut_decode_ranges_round_their_output_once(device, batch, lo, hi, hq, hkv, d, dtype, fused):
+    """A device plan's cut ranges, against one whole unit's accuracy. All scores
+    are 0, so every weight is 1, every product exact, and each output element is
+    the mean of its values: fp32 sums of n values of N(0,1) are off by about
+    2^-24 sqrt(n) on sums of about sqrt(n), far below the rounding step of the
+    16-bit output, and all but a few elements (those within that error of a
+    rounding boundary: under 1% in bf16, 5% in fp16) are the rounded mean.
+    Partial outputs rounded to 16 bits before the merge get a third wrong."""
+    rng = np.random.default_rng(batch)
+    gen = torch.Generator().manual_seed(batch)
+    kv = [int(x) for x in rng.integers(lo, hi, batch)]
+    blocks = sum((n + 15) // 16 for n in kv) + 3
+    tables = random_tables(gen, blocks, kv, 16)
+    kp = torch.randn((blocks, 16, hkv, d), generator=gen).to(dtype).to(device)
+    vp = torch.randn((blocks, 16, hkv, d), generator=gen).to(dtype).to(device)
+    q = torch.zeros((batch, hq, d), dtype=dtype, device=device)
+    plan = nat.plan_attention(list(range(batch + 1)), kv, hq, hkv, d, dtype, device)
+    assert plan.n_merges > 0
+    out = torch.full_like(q, float("nan"))
+    nat.paged_attention(q, out, nat.PoolView.from_bshd(kp, vp), pad_tables(tables, device),
+                        torch.arange(batch + 1, dtype=torch.int32, device=device),
+                        torch.tensor(kv, dtype=torch.int32, device=device),
+                        torch.tensor(kv, dtype=torch.int64, device=device) - 1, plan, d ** -0.5, hkv,
+                        fused_merge=fused)
+    wrong = 0
+    for i, (t, n) in enumerate(zip(tables, kv)):
+        mean = vp[t].reshape(-1, hkv, d)[:n].double().mean(0).to(dtype)
+        wrong += int((out[i].view(hkv, hq // hkv, d) != mean[:, None]).sum())
+    share = wrong / out.numel()
+    assert share <= (0.01 if dtype == torch.bfloat16 else 0.05), share
