@@ -508,7 +508,7 @@ constexpr int coop_lds_bytes() {
 template <int DT, int DP, int NT, bool FAST>
 constexpr int attn_lds_bytes() {
     if constexpr (NT == 1) return coop_lds_bytes<DP>();
-    else return FAST ? wide_lds_bytes<DT, DP>() : 0;
+    else return wide_lds_bytes<DT, DP>();
 }
 
 // The body of one workgroup of the attention kernel: `block` is its index
@@ -1218,6 +1218,15 @@ __device__ __forceinline__ void ld_lds16_base(const char* base_, uint32_t lane_o
 // two score chains at a time took 430 against 436. Scalar registers count too:
 // a base computed for every load apart, with a branch each, took 630 us.
 //
+// Blocks of another size than 16 tokens (BLK16 false) change only where a stage's
+// rows are read from: each lane looks up the block of its own key, one stage
+// ahead. The planner cuts wide work for workgroups that share their tiles and
+// does not see the block size; run wave by wave, its plans took up to 1.7 times
+// as long there as the narrower per-wave ranges of the 16x16 loop. Graph
+// replays, us, 32-token blocks, that loop, wave by wave, and this: 12 verifies
+// of 8 rows at 15/5 heads x 64 33, 50, 20; 6 prompts of up to 900 at 8/2 x 32
+// 24, 39, 13; chunks of 512 and 700 after 2000 and 500 at 40/8 x 128 295, 302, 88.
+//
 // cols holds the first column tile and the tile count of the workgroup's four
 // items, in scalar registers: only the block table's round trip stands before
 // the first stage. Two to three more did -- the other items' columns by vector
@@ -1231,7 +1240,7 @@ __device__ __forceinline__ void ld_lds16_base(const char* base_, uint32_t lane_o
 // (35.8). The wave's own item is read again rather than kept: its registers,
 // held over the caller's comparison, made the 256-byte kernel spill scalars in
 // its loop (two chunks of 2048 rows 409 us against 397).
-template <int DT, int DP, bool TAIL>
+template <int DT, int DP, bool TAIL, bool BLK16>
 __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int block,
                                                const int (&cols)[kWaves][2]) {
     constexpr int RB = DP * 2;       // bytes of one key row
@@ -1259,13 +1268,38 @@ __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int bloc
     const int pool_len = TAIL ? kv_len - nrows : (a.pool_lens != nullptr ? a.pool_lens[s] : kv_len);
 
     // block-table entries of the 64 tiles from tbl_base (one per lane), and of
-    // the 64 after them
+    // the 64 after them (16-token blocks)
     const int32_t* trow = a.block_tables + (int64_t)s * a.bt_stride;
     const int tbl_end = inflight ? min(kt1, (pool_len + 15) >> 4) : kt1;
     const int tbl_last = max(tbl_end - 1, 0);  // tiles past it are new rows: never read through the table
     int tbl_base = kt0;
-    int tbl = trow[min(kt0 + lane, tbl_last)], tbl_next = trow[min(kt0 + 64 + lane, tbl_last)];
+    int tbl = 0, tbl_next = 0;
+    if constexpr (BLK16) {
+        tbl = trow[min(kt0 + lane, tbl_last)];
+        tbl_next = trow[min(kt0 + 64 + lane, tbl_last)];
+    }
     auto tbl_at = [&](int t) -> int { return __builtin_amdgcn_readlane(tbl, t - tbl_base); };  // wave-uniform t
+
+    // other block sizes: the key this lane fetches with its i-th piece of stage u
+    // (clamped to the range and the context, whose last row then stands in: it is
+    // masked there), and the entries of the blocks that hold a stage's keys
+    const unsigned bsz = (unsigned)a.block_size;
+    auto piece_key = [&](int u, int i) -> int {
+        const int x = wave + 4 * i;
+        const int p = x % (2 * PK);
+        const int k16 = (p >= PK ? p - PK : p) * (1024 / RB) + lane * 16 / RB;
+        return min(min(kt0 + TS * u + x / (2 * PK), kt1 - 1) * 16 + k16, kv_len - 1);
+    };
+    auto look = [&](int u, int (&phys)[NLD]) {
+        if constexpr (!BLK16) {
+#pragma unroll
+            for (int i = 0; i < NLD; ++i)
+                phys[i] = trow[(unsigned)max(min(piece_key(u, i), pool_len - 1), 0) / bsz];
+        }
+    };
+    int ph0[NLD], ph1[NLD];
+    look(0, ph0);
+    look(1, ph1);
 
     // ---- this lane's column: position and query (padding columns read
     // row0's and are never stored)
@@ -1325,8 +1359,31 @@ __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int bloc
     // tiles the fetches clamp to: the item's range for the first stage, the
     // workgroup's last read tile once the positions are in
     int fetch_end = kt1;
-    auto fetch = [&](int u, int buf) __attribute__((always_inline)) {
+    auto fetch = [&](int u, int buf, const int (&phys)[NLD]) __attribute__((always_inline)) {
         const int t0 = kt0 + TS * u;
+        if constexpr (!BLK16) {
+#pragma unroll
+            for (int i = 0; i < NLD; ++i) {
+                const int x = wave + 4 * i;
+                const int b = x / (2 * PK), p = x % (2 * PK);
+                const bool isv = p >= PK;
+                const int k16 = (isv ? p - PK : p) * (1024 / RB) + lane * 16 / RB;
+                const int swz = isv ? ((k16 & 3) / RPB) << 2 : (k16 / RPB) & (NCH - 1);
+                const int key = piece_key(u, i);
+                const char* src;
+                if (!inflight || key < pool_len) {
+                    src = k_pool + (isv ? v_delta : 0) + ((int64_t)phys[i] * a.p_sb +
+                                                          (int64_t)((unsigned)key % bsz) * a.p_ss + (int64_t)h * a.p_sh) * 2;
+                } else {
+                    int nr = row0 + key - pool_len;
+                    if (a.row_map) nr = a.row_map[nr];
+                    src = new_k + (isv ? nv_delta : 0) + ((int64_t)nr * a.n_sr + (int64_t)h * a.n_sh) * 2;
+                }
+                ld_lds16(src + (((lane & (NCH - 1)) ^ swz) << 4),
+                         lds_base + (uint32_t)(buf * STG + b * 16 * RB + (isv ? HALF + (p - PK) * 1024 : p * 1024)));
+            }
+            return;
+        }
         if (t0 - tbl_base >= 64) {
             tbl_base += 64;
             tbl = tbl_next;
@@ -1383,7 +1440,7 @@ __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int bloc
         }
     };
     if constexpr (MF_WIDE_PRIO > 0) __builtin_amdgcn_s_setprio(MF_WIDE_PRIO);
-    if (kt1 > kt0) fetch(0, 0);
+    if (kt1 > kt0) fetch(0, 0, ph0);
 
     // ---- the columns' causal limits; tiles past the workgroup's last visible
     // key are not read
@@ -1483,11 +1540,12 @@ __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int bloc
     };
 
     if (nst > 0) {
-        if (nst > 1) fetch(1, 1);
+        if (nst > 1) fetch(1, 1, ph1);
         const int live_end = min(kv_len, wg_end * 16);  // rows past it may hold anything, NaN included
         if (nst > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NLD) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         sync();
+        look(2, ph0);
         for (int u = 0; u < nst; ++u) {
             char* stg = attn_lds + (u & 1) * STG;
             const int key0 = (kt0 + TS * u) * 16;
@@ -1503,7 +1561,10 @@ __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int bloc
                 if (key0 + 32 * v <= maxlim) tile(stg + v * 32 * RB, key0 + 32 * v);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             sync();
-            if (u + 2 < nst) fetch(u + 2, u & 1);
+            if (u + 2 < nst) {
+                fetch(u + 2, u & 1, ph0);
+                look(u + 3, ph0);
+            }
         }
     } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first stage still lands in this workgroup's LDS
@@ -1552,7 +1613,7 @@ __device__ __forceinline__ void attn_wide_body(const AttnArgs& a, const int bloc
 // workgroup's setup (4.0 us alone).
 template <int DT, int DP, int NT, bool FAST, bool TAIL = false>
 __device__ __forceinline__ void attn_block(const AttnArgs& a, const int block) {
-    if constexpr (FAST && DT != MF_F32 && NT > 1) {
+    if constexpr (DT != MF_F32 && NT > 1) {
         const int num_items = a.dev_count ? *a.dev_count : a.num_items;
         const int32_t* i0 = a.items + (int64_t)block * kWaves * MF_PLAN_ITEM_INTS;
         int32_t key[kWaves][4];
@@ -1567,13 +1628,13 @@ __device__ __forceinline__ void attn_block(const AttnArgs& a, const int block) {
             cols[w][0] = iw[2];
             cols[w][1] = iw[3];
         }
-        bool same = (block + 1) * kWaves <= num_items;
+        bool same = (FAST || a.head_dim == DP) & ((block + 1) * kWaves <= num_items);
 #pragma unroll
         for (int w = 1; w < kWaves; ++w)
             same = same & (key[w][0] == key[0][0]) & (key[w][1] == key[0][1]) & (key[w][2] == key[0][2]) &
                    (key[w][3] == key[0][3]);
         if (same) {
-            attn_wide_body<DT, DP, TAIL>(a, block, cols);
+            attn_wide_body<DT, DP, TAIL, FAST>(a, block, cols);
             return;
         }
     }

@@ -32,6 +32,20 @@ def _plan(cu, kv, hq, hkv, d, dtype, dev, cus):
 @pytest.mark.parametrize("cus", [1, 256])  # ranges uncut / cut for a whole device
 @pytest.mark.parametrize("form", ["write", "inflight", "pool"])
 def test_wide_items_match_the_oracle(dtype, hq, hkv, d, cus, form):
+    _against_the_oracle(dtype, hq, hkv, d, cus, form, 16)
+
+
+@pytest.mark.parametrize("bs,dtype", [(1, torch.bfloat16), (8, torch.float16), (12, torch.bfloat16),
+                                      (32, torch.float16), (48, torch.bfloat16)])
+@pytest.mark.parametrize("hq,hkv,d", [(6, 2, 32), (15, 5, 64), (10, 2, 128)])
+@pytest.mark.parametrize("cus", [0, 1, 256])  # 0: the general planner
+@pytest.mark.parametrize("form", ["inflight", "pool"])
+def test_wide_items_on_other_block_sizes_match_the_oracle(bs, dtype, hq, hkv, d, cus, form):
+    """Blocks smaller and larger than a tile, a stage and not a power of two."""
+    _against_the_oracle(dtype, hq, hkv, d, cus, form, bs)
+
+
+def _against_the_oracle(dtype, hq, hkv, d, cus, form, bs):
     dev = torch.device("cuda:0")
     gen = torch.Generator().manual_seed(d + cus)
     # (prior keys, new rows): one tile of columns more than narrow, uneven
@@ -39,7 +53,6 @@ def test_wide_items_match_the_oracle(dtype, hq, hkv, d, cus, form):
     # and past a stage, rows only just wide
     runs = [(0, 64), (2075, 37), (13, 130), (64, 63), (129, 65), (31, 17), (1040, 6)]
     kv = [p + n for p, n in runs]
-    bs = 16
     nblocks = sum((k + bs - 1) // bs for k in kv) + 2
     tables = random_tables(gen, nblocks, kv, bs)
     kp = torch.randn((nblocks, bs, hkv, d), generator=gen).to(dtype)
