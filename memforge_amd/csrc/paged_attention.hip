@@ -2340,15 +2340,15 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
     const int U = mf::kWaves;
     // Decode steps planned for a device (one row a sequence, one column tile
     // each) that the general partition leaves with fewer than two workgroups
-    // per compute unit. There the longest chain of tiles sets the time, so
+    // per compute unit. Where its longest chain of tiles sets the time,
     // ranges run as cooperative units from a few tiles on: above 4 / 16 / 32
     // tiles with up to one / two / more (sequence, kv head) pairs per compute
     // unit, and always above P, the most a single wave of the general partition
     // takes (a longer range left to one wave would also lose its tiles past P;
     // us as four-wave units, then as single waves: 64 sequences of 256 keys at
     // 15/5 heads x 64 6.4, 8.5; 40 of 256 at 40/8 x 128 12.8, 17.9; 120 of up to
-    // 256 at 9/3 x 64 5.1, 8.1). At 256-byte rows a range is cut where the longest holds more than 80
-    // tiles -- below, the merge launch costs more than its chain -- into units of
+    // 256 at 9/3 x 64 5.1, 8.1). At 256-byte rows a range is cut where the
+    // longest holds more than 80 tiles into units of
     // about total / (1.8 x compute units) tiles, at least 32 and at most 72: two
     // workgroups of a unit per compute unit and one round of them. At 128-byte
     // rows, whose tiles chain three times as fast, a step with ranges of more
@@ -2357,10 +2357,27 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
     // Measured, us, general plan then this one: 64 sequences of up to 1152 keys
     // at 15/5 x 64 17.4, 15.3 (units of 64 tiles and merges 19.2); at 40/8 x 128
     // 4 of 8192 to 24576 84, 66 (units of 128 tiles 76, 256 84); 16 of 500 to
-    // 4000 73, 45 (uncut 71); 64 of 200 to 3000 119, 70 (uncut 85). A lone
-    // wave's tile takes 0.33 us at 4 KB of K and V, 0.95 at 8 KB.
+    // 4000 73, 45 (uncut 71); 64 of 200 to 3000 119, 70 (uncut 85).
+    //
+    // Which plan takes less time is estimated from the longest chain one wave
+    // runs (a tile takes 0.33 us at 4 KB of K and V, 0.95 at 8 KB and in
+    // proportion above), the bytes at 5.5 TB/s, and a merge launch of 4 us. Where
+    // the bytes set the general plan's time and the two come out about the same,
+    // the general plan is kept if its workgroups fill the compute units evenly
+    // (its tiles are at least 0.7 of those that every unit's longest would make);
+    // else its last workgroups run on a part-empty chip. Graph replays over pools
+    // larger than the caches, us, general plan then this one whatever the
+    // estimate: 1 sequence of 1400 keys at 9/3 x 64 8.7, 11.0; 4 of 1400 at 15/5
+    // x 64 8.9, 11.0; 2 of about 2000 at 40/8 x 128 13.6, 16.8; 100 of 1400 there
+    // 105, 128 (even), 33 of 5000 202, 128 (264 workgroups on 256 units). Over
+    // 772 steps of 1 to 200 sequences at seven shapes the choice takes 0.1% more
+    // than the better plan on average, and 8 take over 5% more.
     int single_max = P;
     double unit_tiles = 0;  // tiles per unit of a cut range (0: the general partition)
+    const auto decode_units = [](int tiles, double per_unit) {
+        const int n = std::max(1, (int)std::lround(tiles / per_unit));
+        return std::max(n, (tiles + mf::kWaves * mf::kMaxItemTiles - 1) / (mf::kWaves * mf::kMaxItemTiles));
+    };
     if (num_cus > 0 && partition_tiles <= 0 && !mixed) {
         int64_t pairs = 0, tiles_all = 0, singles = 0, units = 0;
         int longest = 0;
@@ -2376,20 +2393,46 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
             if (T > P) units += (int64_t)Hkv * ((T + U * P - 1) / (U * P));
             else singles += Hkv;
         }
-        if (decode && units + singles / U < 2 * (int64_t)num_cus) {
-            const bool long_rows = DP * mf::dtype_size(dtype) >= 256;
-            if (long_rows || longest <= 100) {
-                single_max = std::min(P, pairs <= num_cus ? 4 : pairs <= 2 * (int64_t)num_cus ? 16 : 32);
-                unit_tiles = long_rows && longest > 80
-                                 ? std::min(72.0, std::max(32.0, (double)tiles_all / (1.8 * num_cus)))
-                                 : 1e9;
+        const int row_bytes = DP * mf::dtype_size(dtype);
+        const bool long_rows = row_bytes >= 256;
+        if (decode && units + singles / U < 2 * (int64_t)num_cus && (long_rows || longest <= 100)) {
+            const int single = std::min(P, pairs <= num_cus ? 4 : pairs <= 2 * (int64_t)num_cus ? 16 : 32);
+            const double per_unit = long_rows && longest > 80
+                                        ? std::min(72.0, std::max(32.0, (double)tiles_all / (1.8 * num_cus)))
+                                        : 1e9;
+            const double tile_us = row_bytes >= 256 ? 0.95 * row_bytes / 256 : 0.33;
+            const double bytes_us = (double)tiles_all * 32 * row_bytes / 5.5e6;
+            struct Shape {
+                double chain_us, us;  // the longest chain's time, the estimate
+                double fill;          // tiles over those of a grid of longest workgroups
+            };
+            auto shape = [&](int alone, auto units_of) {
+                int chain = 0, work = 0;
+                int64_t waves = 0;
+                bool split = false;
+                for (int s = 0; s < num_seqs; ++s) {
+                    if (!col_tiles(s)) continue;
+                    const int T = (kv_lens[s] + 15) / 16;
+                    const int n = T <= alone ? 1 : units_of(T);
+                    const int unit = (T + n - 1) / n;
+                    chain = std::max(chain, T <= alone ? T : (unit + U - 1) / U);
+                    work = std::max(work, T <= alone ? U * T : unit);
+                    waves += (int64_t)Hkv * (T <= alone ? 1 : U * n);
+                    split = split || n > 1;
+                }
+                const int64_t grid = ((waves + U - 1) / U + num_cus - 1) / num_cus * num_cus;
+                return Shape{chain * tile_us, std::max(bytes_us, chain * tile_us) + (split ? 4.0 : 0.0),
+                             (double)tiles_all / ((double)grid * std::max(work, 1))};
+            };
+            const Shape general = shape(P, [&](int T) { return (T + U * P - 1) / (U * P); });
+            const Shape units_only = shape(single, [&](int T) { return decode_units(T, per_unit); });
+            if (units_only.us < 0.995 * general.us ||
+                (units_only.us <= 1.2 * general.us && bytes_us >= 0.9 * general.chain_us && general.fill < 0.7)) {
+                single_max = single;
+                unit_tiles = per_unit;
             }
         }
     }
-    auto decode_units = [&](int tiles) {
-        const int n = std::max(1, (int)std::lround(tiles / unit_tiles));
-        return std::max(n, (tiles + U * mf::kMaxItemTiles - 1) / (U * mf::kMaxItemTiles));
-    };
     auto round_up = [&](int64_t n) { return (n + U - 1) / U * U; };
     // key partitions of sequence s: count, and the start of partition p
     // (narrow cooperative ranges are balanced; the rest are Q-tile strides).
@@ -2401,7 +2444,7 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
         const int tiles = (kv_lens[s] + 15) / 16;
         coop = narrow && tiles > single_max;
         Q = narrow ? (coop ? U * P : P) : PW;
-        if (narrow && unit_tiles > 0) return coop ? decode_units(tiles) : 1;
+        if (narrow && unit_tiles > 0) return coop ? decode_units(tiles, unit_tiles) : 1;
         if (!narrow && tiles > PW) {
             const int np = (tiles + PW - 1) / PW;
             Q = (tiles + np - 1) / np;

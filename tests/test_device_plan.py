@@ -139,3 +139,17 @@ def test_single_column_items_fit_their_block_table_registers(cus, partition, hq,
         narrow = made[0][:int(made[2][0])]
         assert narrow.shape[0] and int((narrow[:, 5] - narrow[:, 4]).max()) <= nat.MAX_ITEM_TILES, tiles
         _cover(*made, [rows] * 32, kv, hq, hkv, d)
+
+
+@pytest.mark.parametrize("heads,kv,kept", [
+    ((9, 3, 64), [1400], True), ((15, 5, 64), [1400] * 4, True), ((40, 8, 128), [1772, 2171], True),  # short chains
+    ((40, 8, 128), [1400] * 100, True),                                       # bytes, and an even grid
+    ((40, 8, 128), [5000] * 33, False),                                       # bytes, 264 workgroups on 256 units
+    ((15, 5, 64), [40 + 18 * i for i in range(64)], False), ((40, 8, 128), [8192, 12000, 20000, 24576], False),
+])
+def test_device_decode_rule_gives_way_where_the_general_plan_is_the_shorter(heads, kv, kept):
+    cu = list(range(len(kv) + 1))
+    a = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16, num_cus=256)
+    b = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16)
+    assert all(np.array_equal(x, y) for x, y in zip(a, b)) == kept
+    _cover(*a, [1] * len(kv), kv, *heads)
