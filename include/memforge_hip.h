@@ -368,6 +368,17 @@ int mf_attention_plan_device(int num_seqs, const int32_t* cu_seqlens, const int3
                              int32_t* items, int64_t items_capacity, int32_t* merges,
                              int64_t merges_capacity, int64_t* counts);
 
+/* mf_attention_plan_device for a launch that has no merge behind it (a captured
+ * decode step): its decode units hold whole ranges, up to 512 tiles. A plan
+ * that still has merges (counts[2]) is the general planner's, where no such
+ * units were the better choice; the caller then plans with partition_tiles, the
+ * smallest power of two from 4 whose units (four times as many tiles) hold the
+ * longest range. No counterpart in the reference. */
+int mf_attention_plan_merge_free(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
+                                 int num_q_heads, int num_kv_heads, int head_dim, int dtype, int num_cus,
+                                 int32_t* items, int64_t items_capacity, int32_t* merges,
+                                 int64_t merges_capacity, int64_t* counts);
+
 /* ------------------------------------------------- decode slice plans
  * A second plan form for large decode launches, with the same results as
  * mf_attention_plan + mf_paged_attention (up to fp32 summation order).

@@ -77,6 +77,8 @@ _SIGNATURES = {
                                    _vp, _c_i64, _vp, _c_i64, _vp]),
     "mf_attention_plan_device": (_c_int, [_c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int,
                                           _vp, _c_i64, _vp, _c_i64, _vp]),
+    "mf_attention_plan_merge_free": (_c_int, [_c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                              _vp, _c_i64, _vp, _c_i64, _vp]),
     "mf_attention_plan_slices": (_c_int, [_c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int,
                                           _c_int, _vp, _c_i64, _vp, _c_i64, _vp]),
     "mf_paged_attention_slices": (_c_int, [
@@ -406,11 +408,13 @@ class AttentionPlan:
 
 def plan_attention_host(cu_seqlens: Sequence[int], kv_lens: Sequence[int], num_q_heads: int,
                         num_kv_heads: int, head_dim: int, dtype: torch.dtype,
-                        partition_tiles: int = 0, num_cus: int = 0) -> Tuple[np.ndarray, np.ndarray, np.ndarray]:
+                        partition_tiles: int = 0, num_cus: int = 0,
+                        merge_free: bool = False) -> Tuple[np.ndarray, np.ndarray, np.ndarray]:
     """mf_attention_plan on host arrays: (items [n, PLAN_ITEM_INTS], merges
     [m, PLAN_MERGE_INTS], counts [n_narrow, n_wide, n_merges, partials_floats]).
     With ``num_cus`` and no ``partition_tiles``, mf_attention_plan_device: the
-    ranges cut for a GPU of that many compute units."""
+    ranges cut for a GPU of that many compute units; with ``merge_free`` as well,
+    mf_attention_plan_merge_free, which does not cut decode ranges for it."""
     cu = np.ascontiguousarray(np.asarray(cu_seqlens, dtype=np.int32))
     kv = np.ascontiguousarray(np.asarray(kv_lens, dtype=np.int32))
     B = kv.shape[0]
@@ -420,7 +424,8 @@ def plan_attention_host(cu_seqlens: Sequence[int], kv_lens: Sequence[int], num_q
     L = lib()
     args = [B, cu.ctypes.data, kv.ctypes.data, num_q_heads, num_kv_heads, head_dim, dtype_code(dtype)]
     device = num_cus > 0 and partition_tiles <= 0
-    plan = L.mf_attention_plan_device if device else L.mf_attention_plan
+    plan = L.mf_attention_plan if not device else \
+        L.mf_attention_plan_merge_free if merge_free else L.mf_attention_plan_device
     args.append(num_cus if device else partition_tiles)
     # One planner call when the plan fits the largest one seen so far (the
     # planner fills every row it reports); otherwise it reports the sizes and

@@ -2190,9 +2190,10 @@ inline int part_dstride_for(int head_dim) { return head_dim < 32 ? 32 : head_dim
 }  // namespace mf
 
 namespace {
-// The planner of mf_attention_plan (num_cus 0) and mf_attention_plan_device.
+// The planner of mf_attention_plan (num_cus 0), mf_attention_plan_device and
+// mf_attention_plan_merge_free (cut false).
 int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens, int num_q_heads,
-                   int num_kv_heads, int head_dim, int dtype, int partition_tiles, int num_cus, int32_t* items,
+                   int num_kv_heads, int head_dim, int dtype, int partition_tiles, int num_cus, bool cut, int32_t* items,
                    int64_t items_capacity, int32_t* merges, int64_t merges_capacity, int64_t* counts) {
     if (num_seqs < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || !counts)
         return MF_ERR_ARG;
@@ -2397,7 +2398,7 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
         const bool long_rows = row_bytes >= 256;
         if (decode && units + singles / U < 2 * (int64_t)num_cus && (long_rows || longest <= 100)) {
             const int single = std::min(P, pairs <= num_cus ? 4 : pairs <= 2 * (int64_t)num_cus ? 16 : 32);
-            const double per_unit = long_rows && longest > 80
+            const double per_unit = cut && long_rows && longest > 80
                                         ? std::min(72.0, std::max(32.0, (double)tiles_all / (1.8 * num_cus)))
                                         : 1e9;
             const double tile_us = row_bytes >= 256 ? 0.95 * row_bytes / 256 : 0.33;
@@ -2405,6 +2406,7 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
             struct Shape {
                 double chain_us, us;  // the longest chain's time, the estimate
                 double fill;          // tiles over those of a grid of longest workgroups
+                bool split;
             };
             auto shape = [&](int alone, auto units_of) {
                 int chain = 0, work = 0;
@@ -2422,9 +2424,16 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
                 }
                 const int64_t grid = ((waves + U - 1) / U + num_cus - 1) / num_cus * num_cus;
                 return Shape{chain * tile_us, std::max(bytes_us, chain * tile_us) + (split ? 4.0 : 0.0),
-                             (double)tiles_all / ((double)grid * std::max(work, 1))};
+                             (double)tiles_all / ((double)grid * std::max(work, 1)), split};
             };
-            const Shape general = shape(P, [&](int T) { return (T + U * P - 1) / (U * P); });
+            Shape general = shape(P, [&](int T) { return (T + U * P - 1) / (U * P); });
+            if (!cut && general.split) {
+                // the plan a merge-free launch gets without the rule: the smallest
+                // partition whose units hold the longest range whole
+                int q = 4;
+                while (U * q < longest && q < mf::kMaxItemTiles) q *= 2;
+                general = shape(q, [&](int T) { return (T + U * q - 1) / (U * q); });
+            }
             const Shape units_only = shape(single, [&](int T) { return decode_units(T, per_unit); });
             if (units_only.us < 0.995 * general.us ||
                 (units_only.us <= 1.2 * general.us && bytes_us >= 0.9 * general.chain_us && general.fill < 0.7)) {
@@ -2913,7 +2922,7 @@ extern "C" int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const 
                                  int partition_tiles, int32_t* items, int64_t items_capacity,
                                  int32_t* merges, int64_t merges_capacity, int64_t* counts) {
     return attention_plan(num_seqs, cu_seqlens, kv_lens, num_q_heads, num_kv_heads, head_dim, dtype,
-                          partition_tiles, 0, items, items_capacity, merges, merges_capacity, counts);
+                          partition_tiles, 0, true, items, items_capacity, merges, merges_capacity, counts);
 }
 
 extern "C" int mf_attention_plan_device(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
@@ -2921,7 +2930,16 @@ extern "C" int mf_attention_plan_device(int num_seqs, const int32_t* cu_seqlens,
                                         int32_t* items, int64_t items_capacity, int32_t* merges,
                                         int64_t merges_capacity, int64_t* counts) {
     if (num_cus <= 0) return MF_ERR_ARG;
-    return attention_plan(num_seqs, cu_seqlens, kv_lens, num_q_heads, num_kv_heads, head_dim, dtype, 0, num_cus,
+    return attention_plan(num_seqs, cu_seqlens, kv_lens, num_q_heads, num_kv_heads, head_dim, dtype, 0, num_cus, true,
+                          items, items_capacity, merges, merges_capacity, counts);
+}
+
+extern "C" int mf_attention_plan_merge_free(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
+                                            int num_q_heads, int num_kv_heads, int head_dim, int dtype,
+                                            int num_cus, int32_t* items, int64_t items_capacity, int32_t* merges,
+                                            int64_t merges_capacity, int64_t* counts) {
+    if (num_cus <= 0) return MF_ERR_ARG;
+    return attention_plan(num_seqs, cu_seqlens, kv_lens, num_q_heads, num_kv_heads, head_dim, dtype, 0, num_cus, false,
                           items, items_capacity, merges, merges_capacity, counts);
 }
 

@@ -194,7 +194,8 @@ class GraphedPagedDecoder:
         kv = [int(c) + 1 for c in ctx_lens] + [0] * (b - n)
         plan_args = (list(range(b + 1)), kv, self.num_q_heads, self.pool.spec.num_kv_heads,
                      self.pool.spec.head_dim, self.pool.key_pool.dtype)
-        items, merges, counts = nat.plan_attention_host(*plan_args, num_cus=nat.device_cus(self.device))
+        items, merges, counts = nat.plan_attention_host(*plan_args, num_cus=nat.device_cus(self.device),
+                                                        merge_free=self.merge_free)
         if self.merge_free and counts[2] > 0:
             # the planner's pick splits a range: take the smallest partition
             # whose units hold the longest context whole instead

@@ -153,3 +153,19 @@ def test_device_decode_rule_gives_way_where_the_general_plan_is_the_shorter(head
     b = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16)
     assert all(np.array_equal(x, y) for x, y in zip(a, b)) == kept
     _cover(*a, [1] * len(kv), kv, *heads)
+
+
+@pytest.mark.parametrize("heads", [(40, 8, 128), (15, 5, 64)])
+def test_merge_free_plans_hold_whole_ranges(heads):
+    rng = np.random.default_rng(9)
+    taken = 0
+    for kv in ([int(x) for x in rng.integers(200, 3000, 64)], [8176, 1000, 1000], [8192] * 4, [1500] * 8, [300] * 20,
+               [40 + 18 * i for i in range(64)], [9000] * 2):
+        cu = list(range(len(kv) + 1))
+        made = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16, num_cus=256, merge_free=True)
+        _cover(*made, [1] * len(kv), kv, *heads)
+        general = nat.plan_attention_host(cu, kv, *heads, torch.bfloat16)
+        if not all(np.array_equal(x, y) for x, y in zip(made, general)):
+            assert made[1].shape[0] == 0 and max(kv) <= 8192
+            taken += 1
+    assert taken >= (3 if heads[2] == 128 else 1)

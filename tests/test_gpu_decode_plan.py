@@ -127,3 +127,40 @@ def test_cut_decode_ranges_round_their_output_once(device, batch, lo, hi, hq, hk
         wrong += int((out[i].view(hkv, hq // hkv, d) != mean[:, None]).sum())
     share = wrong / out.numel()
     assert share <= (0.01 if dtype == torch.bfloat16 else 0.05), share
+
+
+def test_graphed_decoder_plans_a_merge_free_step_once(device, monkeypatch):
+    """Ranges that a device plan would cut (256-byte rows and more, over 80
+    tiles): the merge-free decoder asks once, for whole ranges, and runs them as
+    cooperative units; against transformers' attention."""
+    from transformers.cache_utils import DynamicCache
+
+    from memforge_amd.runtime.graphed_paged_decode import GraphedPagedDecoder
+    from memforge_amd.runtime.kv_pool import ModelKVSpec, PagedKVPool
+
+    ctx, tokens = [2100, 1000, 999], [9, 12, 40]
+    model = tiny_llama(num_layers=1, heads=4, kv_heads=2, head_dim=128)
+    blocks = sum((c + 16) // 16 for c in ctx) + 2
+    pool = PagedKVPool(ModelKVSpec.from_config(model.config, torch.float32, "cuda:0"), blocks, 16)
+    gen = torch.Generator().manual_seed(4)
+    pool.key_pool.copy_(torch.randn(pool.key_pool.shape, generator=gen).to(device))
+    pool.value_pool.copy_(torch.randn(pool.value_pool.shape, generator=gen).to(device))
+    tables = random_tables(gen, blocks, [c + 1 for c in ctx], 16)
+    want = []
+    for t, c, tok in zip(tables, ctx, tokens):
+        slots = torch.tensor([t[p // 16] * 16 + p % 16 for p in range(c)], device=device)
+        cache = DynamicCache()
+        cache.update(*(p[0].reshape(-1, 2, 128)[slots].transpose(0, 1).unsqueeze(0).contiguous()
+                       for p in (pool.key_pool, pool.value_pool)), 0)
+        with torch.no_grad():
+            want.append(model(input_ids=torch.tensor([[tok]], device=device),
+                              position_ids=torch.tensor([[c]], device=device), past_key_values=cache,
+                              use_cache=True).logits[0, -1])
+    made = []
+    plan = nat.plan_attention_host
+    monkeypatch.setattr(nat, "plan_attention_host", lambda *a, **kw: made.append(plan(*a, **kw)) or made[-1])
+    dec = GraphedPagedDecoder(model, pool, max_batch=4, max_model_len=2200)
+    assert dec.merge_free
+    for _ in range(3):
+        torch.testing.assert_close(dec.step(tokens, ctx, tables), torch.stack(want), atol=2e-5, rtol=1e-4)
+    assert len(made) == 3 and all((items[:, 11] == 1).all() and counts[2] == 0 for items, _, counts in made)
