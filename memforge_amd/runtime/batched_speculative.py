@@ -424,6 +424,7 @@ def resolve_rounds_batched(seq_ids: Sequence[int], candidates: torch.Tensor, dra
     """
     # the candidates' copy is queued ahead of the kernels and the four results
     # come back as the one buffer they share, so the host waits once
+    nat.require_device(candidates)
     cand_host = torch.empty(candidates.shape, dtype=candidates.dtype, pin_memory=True)
     cand_host.copy_(candidates, non_blocking=True)
     packed = nat.spec_verify(candidates, draft_probs, target_logits, temperature, u_accept, exp_noise).packed.cpu()

@@ -59,3 +59,13 @@ def test_varlen_launcher_reads_only_the_pool_part_of_a_verify_table():
 def test_pool_view_bounds():
     pool = _pool(num_blocks=5, bs=16)
     assert pool.num_blocks == 5 and pool.num_slots == 80
+
+
+def test_batched_rejection_refuses_host_tensors_before_it_pins_memory():
+    """Candidates in host memory are the caller's mistake, named as such also
+    where no GPU is there to pin memory for."""
+    from memforge_amd.runtime.batched_speculative import resolve_rounds_batched
+
+    with pytest.raises(ValueError, match="runs on the GPU"):
+        resolve_rounds_batched(range(2), torch.zeros((2, 1), dtype=torch.int32), torch.rand(2, 1, 8),
+                               torch.rand(2, 2, 8), 1.0, torch.rand(2, 1), torch.rand(2, 8))
