@@ -357,12 +357,16 @@ int mf_attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv
 
 /* mf_attention_plan for a device of `num_cus` compute units
  * (hipDeviceProp_t::multiProcessorCount), with the partitions chosen by the
- * planner: the same records, run by the same entry points, with the same
- * results up to fp32 summation order. Wide workgroups (16-bit types, head_dim
+ * planner: the same records, run by the same entry points. Ranges are cut
+ * elsewhere than in mf_attention_plan, so the results are those of another
+ * summation order; a partial output is one rounding to the launch's type,
+ * except where decode ranges are cut that the other planner leaves whole
+ * (MF_PLAN_FP32_PARTIALS). Wide workgroups (16-bit types, head_dim
  * a kernel size) are cut by column quads, for about two or four workgroups per
  * compute unit, with ranges of any length; decode rows that leave compute
- * units idle run as more and shorter cooperative units. No counterpart
- * in the reference: it serves the launch, not the data path. */
+ * units idle run as more and shorter cooperative units where that takes less
+ * time. No counterpart in the reference: it serves the launch, not the data
+ * path. */
 int mf_attention_plan_device(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_lens,
                              int num_q_heads, int num_kv_heads, int head_dim, int dtype, int num_cus,
                              int32_t* items, int64_t items_capacity, int32_t* merges,

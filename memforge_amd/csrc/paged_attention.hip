@@ -18,9 +18,10 @@
 // A layout with byte permutes. 16-bit prefill runs in workgroups that share
 // each K/V row through LDS instead (attn_wide_body).
 //
-// Long contexts are split into key partitions (the plan decides); partial
-// (max, sum, unnormalised output) triples go to fp32 scratch and a merge
-// kernel combines them with the log-sum-exp rule.
+// Long contexts are split into key partitions (the plan decides); each leaves
+// its running maximum and sum in fp32 and its normalised output in the launch's
+// type (or in fp32, see the split-K merge), and a merge kernel combines them
+// with the log-sum-exp rule.
 #include <algorithm>
 #include <array>
 #include <atomic>
@@ -446,7 +447,11 @@ __device__ __forceinline__ void arrive_and_merge(const AttnArgs& a, int m0, int 
 // -------------------------------------------------------------- main kernel
 // Waves per SIMD the register allocator must leave room for: two where the
 // kernel fits in 256 registers without spilling (key rows up to 128 bytes,
-// or up to 256 bytes for single-tile items), else one.
+// or up to 256 bytes for single-tile items), else one. 16-bit wide kernels are
+// held to what the shared loop gains from, four (three at 256-byte rows). There
+// the whole kernel, with the wave-by-wave body beside the loop, spills at 168
+// registers: 61 to 67 vector and 24 to 32 scalar ones, 236 to 244 bytes of
+// scratch, most of them the wave-by-wave body's.
 #ifndef MF_WIDE_WAVES
 #define MF_WIDE_WAVES(dp) ((dp) == 128 ? 3 : 4)
 #endif
@@ -1197,8 +1202,8 @@ __device__ __forceinline__ void ld_lds16_base(const char* base_, uint32_t lane_o
 // registers as they are, and V^T's A operand is read in the same key order by
 // the transposing LDS read, so neither P nor V moves between lanes.
 //
-// Stages of 64 keys go from global memory straight into LDS (two buffers, one
-// barrier per stage). Each wave loads the same few 1 KB pieces of every
+// Stages of 64 keys (32 at 256-byte rows) go from global memory straight into
+// LDS (two buffers, one barrier per stage). Each wave loads the same few 1 KB pieces of every
 // 16-key block, so a piece is one scalar base plus a lane offset that never
 // changes: new rows of a written-in-flight step are just another base and
 // offset. K rows are xor-swizzled by key in 16-byte chunks (32 keys x one
@@ -1214,7 +1219,8 @@ __device__ __forceinline__ void ld_lds16_base(const char* base_, uint32_t lane_o
 // rather than together -- timing copies without the exponentials, the PV
 // products or the LDS reads each gained 10-25%, none more. So waves per SIMD
 // count: at 256-byte rows 32-key stages leave room for three (168 registers,
-// 32 KB of LDS a workgroup), 373 us against 403 with two and 64-key stages;
+// with spills, and 32 KB of LDS a workgroup), 373 us against 403 with two and
+// 64-key stages;
 // two score chains at a time took 430 against 436. Scalar registers count too:
 // a base computed for every load apart, with a branch each, took 630 us.
 //
@@ -2474,9 +2480,9 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
     // beside the narrow ones, all in one resident round. C2 step, engine
     // layer as graph replays: 44.1-44.2 us against 45.8-46.0 with the ranges'
     // partitions (PW 64 strides); 1.5 workgroups per CU 49.3-49.6, 2.5
-    // 47.1-47.4, 3 47.5-48.0, 4 53.3-53.5. Plans of wide items only keep the
-    // ranges' partitions (there two per CU took the prefill items from 35.1
-    // to 37.9 us). The XCD queues below take a (sequence, kv head)'s quads
+    // 47.1-47.4, 3 47.5-48.0, 4 53.3-53.5. Plans of wide items only, made without
+    // a device, keep the ranges' partitions (there two per CU took the prefill
+    // items of the 16x16 loop from 35.1 to 37.9 us). The XCD queues below take a (sequence, kv head)'s quads
     // as one run: the launch fetches 1.09x its algorithmic reads, against
     // 1.65x with each (quad, kv head) dealt alone (0.3 us faster).
     const int kPlanCUs = num_cus > 0 ? num_cus : 256;  // an MI355X has 256 compute units
