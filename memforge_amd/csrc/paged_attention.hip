@@ -450,8 +450,9 @@ __device__ __forceinline__ void arrive_and_merge(const AttnArgs& a, int m0, int 
 // or up to 256 bytes for single-tile items), else one. 16-bit wide kernels are
 // held to what the shared loop gains from, four (three at 256-byte rows). There
 // the whole kernel, with the wave-by-wave body beside the loop, spills at 168
-// registers: 61 to 67 vector and 24 to 32 scalar ones, 236 to 244 bytes of
-// scratch, most of them the wave-by-wave body's.
+// registers: 61 to 67 vector and 22 to 24 scalar ones, 236 to 244 bytes of
+// scratch (50 to 55 vector ones on other block sizes than 16). Compiled without
+// that body the loop spills 1 or 2 (9).
 #ifndef MF_WIDE_WAVES
 #define MF_WIDE_WAVES(dp) ((dp) == 128 ? 3 : 4)
 #endif
