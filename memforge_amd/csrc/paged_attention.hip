@@ -2516,9 +2516,15 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
     double quad_w = 1.0;
     const int max_range = device ? INT_MAX : mf::kMaxItemTiles;
     if (mixed || device) {
-        int64_t visible = 0;
+        int64_t visible = 0, quad_units = 0;
+        int longest = 0;
         for (int s = 0; s < num_seqs; ++s)
-            for (int qd = 0, nq = quads(s); qd < nq; ++qd) visible += (int64_t)Hkv * quad_visible(s, qd);
+            for (int qd = 0, nq = quads(s); qd < nq; ++qd) {
+                const int v = quad_visible(s, qd);
+                visible += (int64_t)Hkv * v;
+                quad_units += Hkv;
+                longest = std::max(longest, v);
+            }
         quad_w = std::max((double)std::max(PW, 1), (double)visible / (2.0 * kPlanCUs));
         if (device && !mixed) {
             // About two workgroups per compute unit, of at least 16 tiles (12 at
@@ -2532,7 +2538,20 @@ int attention_plan(int num_seqs, const int32_t* cu_seqlens, const int32_t* kv_le
             // 50 / 36 / 36 / 41 / 45 uncut (20); 2 chunks of about 850 rows
             // after 4000 keys x 128 714 / 449 / 374 / 335 / 301 / 291 / 295 / 292
             // (200: 284).
-            quad_w = std::max(DP >= 128 ? 12.0 : 16.0, (double)visible / (2.0 * kPlanCUs));
+            // Short launches: cut in two, their quads run half the chain and
+            // then a merge, which costs more than the other half. Whole quads
+            // where the longest sees at most 31 tiles; where the (quad, kv head)
+            // pairs fill no more than a third of the compute units, at most 21,
+            // and above that, up to 95, ranges of 8 tiles that the idle units
+            // run beside each other. Graph replays over pools larger than the
+            // caches, us at 8 tiles / the floor above / whole: 8-row verifies of
+            // up to 450 keys at 15/5 heads x 64, 3 of them 9.9 / 10.2 / 10.2, 16
+            // 11.9 / 14.5 / 12.8, 40 12.9 / 14.8 / 12.5; of up to 1000, 8 of them
+            // 12.3 / 14.0 / 20; 16 prompts of up to 500 at 9/3 x 64 18.1 / 17.4 /
+            // 15.2; 4 of up to 300 at 40/8 x 128 22.7 / 22.4 / 19.0.
+            const bool few = quad_units <= kPlanCUs / 3;
+            const double floor = longest < (few ? 22 : 32) ? longest : few && longest < 96 ? 8 : DP >= 128 ? 12 : 16;
+            quad_w = std::max(floor, (double)visible / (2.0 * kPlanCUs));
             if (quad_w > 96) quad_w = std::max(96.0, (double)visible / (4.0 * kPlanCUs));
         }
     }

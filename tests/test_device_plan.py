@@ -169,3 +169,16 @@ def test_merge_free_plans_hold_whole_ranges(heads):
             assert made[1].shape[0] == 0 and max(kv) <= 8192
             taken += 1
     assert taken >= (3 if heads[2] == 128 else 1)
+
+
+@pytest.mark.parametrize("seqs,keys,rows,parts", [
+    (3, 330, 8, 1),                  # few workgroups, 21 tiles: whole
+    (3, 450, 8, 4), (16, 440, 8, 4),  # few workgroups: ranges of about 8 tiles
+    (40, 490, 8, 1),                 # more workgroups, 31 tiles: whole
+    (40, 1000, 8, 3),                # more, and enough work for two workgroups a compute unit
+])
+def test_short_wide_launches_are_cut_finely_or_not_at_all(seqs, keys, rows, parts):
+    cu, kv = [rows * i for i in range(seqs + 1)], [keys] * seqs
+    made = nat.plan_attention_host(cu, kv, 15, 5, 64, torch.bfloat16, num_cus=256)
+    _cover(*made, [rows] * seqs, kv, 15, 5, 64)
+    assert int(made[2][0]) == 0 and int(made[2][1]) == 4 * 5 * seqs * parts
